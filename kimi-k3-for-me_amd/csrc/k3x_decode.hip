@@ -96,22 +96,6 @@ struct KSLds {
     alignas(16) double pl[NT / WAVE][KS_CH];     // ks_chain's products
 };
 
-// The choice key (choice_key's order) just above choice + slack: an upper bound of the
-// reference's choice for an expert whose logit is not proven.
-__device__ __forceinline__ uint32_t slack_key(float choice, float slack)
-{
-    const uint32_t k = choice_key((float)((double)choice + (double)slack));
-    return (k != 0u && k < 0xFF800000u) ? k + 1u : k;
-}
-
-// Whether an expert not proven could change a selection whose K-th choice is ck, or one
-// of its weights: its choice may reach ck (hk: the token's largest slack_key, 0 = none).
-// Every selected expert's choice is at least ck, so a selected one not proven counts.
-__device__ __forceinline__ bool slack_reaches(uint32_t hk, float ck)
-{
-    return hk != 0u && hk >= choice_key(ck);
-}
-
 // The logit of (token t, expert e) as the reference computes it: one double chain
 // acc += (double)W[e][i] * (double)x[i] for i = 0 .. H-1 in order (k3_ops.c:1666-1688),
 // with x the row the router read (nw[i] * x[i] * inv for the RMSNorm of x).  The whole
@@ -486,18 +470,16 @@ __device__ void k1_norm_inv(const K1Args &a, float *lds, float *s_inv)
 // shuffle tree, the four waves' pairs), so the reference's logit is a double within
 // d = chain_gap of v, and its float lies in [(float)(v - d), (float)(v + d)]; where both
 // ends round to (float)v, the float logit, and with it the score and the choice, are the
-// reference's, and the slack is 0.  Otherwise the slack bounds the distance of the
-// reference's choice from this one: a quarter of the float interval's half-width (the
-// sigmoid's slope is at most 1/4) plus the roundings of the sigmoid and of the bias add (a
-// few units in the last place of |choice| <= 2 + |bias|).  NaN logits give a NaN slack,
-// which marks nothing (a NaN choice is never selected, here or in the reference).
+// reference's, and the slack is 0.  Otherwise logit_slack of that interval.  NaN logits give
+// a NaN slack, which marks nothing (a NaN choice is never selected, here or in the
+// reference).
 __device__ __forceinline__ float choice_slack(double v, float asum, int H, float bias)
 {
     const double d = chain_gap(abs_bound(asum, H), H);
     const float f = (float)v, lo = (float)(v - d), hi = (float)(v + d);
     if (lo == f && hi == f) return 0.0f;
     const double df = fmax((double)hi - (double)f, (double)f - (double)lo);
-    return (float)((df * 0.25 + (2.0 + fabs((double)bias)) * 0x1p-21) * 1.01);
+    return logit_slack(df, bias);
 }
 
 // A thread's RCH chunks of four activations of one row (chunk c: elements 4f .. 4f + 3,

@@ -103,7 +103,8 @@ typedef struct k3x_prefill_buf {
     int       nretired;
     size_t    retired_bytes;
     uint16_t *xhl;          /* [T][H/8][2][8] bf16 hi/lo activation rows            */
-    float    *score, *choice; /* [T][E]                                             */
+    float    *logit, *gap;  /* [T][E] router logits, and how far the reference's can lie
+                               from each (0: equal)                                   */
     int      *idx;          /* [T][K]                                                */
     float    *wt;           /* [T][K]                                                */
     int      *counts;       /* [E] tokens per expert                                 */

@@ -965,7 +965,7 @@ size_t k3x_pf_layout(const k3x_moe_layer *L, int T, char *p, k3x_prefill_buf *B)
     const int ndd = (int)(((H + 63) / 64) * (t * K / 16 + E + 1));
     const size_t sz[] = {
         t * H * 4,                 /* xhl     */
-        t * E * 4, t * E * 4,      /* score, choice */
+        t * E * 4, t * E * 4,      /* logit, gap */
         t * K * 4, t * K * 4,      /* idx, wt */
         E * 4, (E + 1) * 4, E * 4, /* counts, offsets, cursor */
         2 * (E + 1) * 4, 2 * (E + 1) * 4,  /* tb_gu, tb_dn: small and large tile classes */
@@ -988,7 +988,7 @@ size_t k3x_pf_layout(const k3x_moe_layer *L, int T, char *p, k3x_prefill_buf *B)
     if (!p || !B) return total;
     B->bytes = total; B->cap_T = T;
     B->xhl = (uint16_t *)(p + off[0]);
-    B->score = (float *)(p + off[1]);   B->choice = (float *)(p + off[2]);
+    B->logit = (float *)(p + off[1]);   B->gap = (float *)(p + off[2]);
     B->idx = (int *)(p + off[3]);       B->wt = (float *)(p + off[4]);
     B->counts = (int *)(p + off[5]);    B->offsets = (int *)(p + off[6]);
     B->cursor = (int *)(p + off[7]);

@@ -1,10 +1,12 @@
 // k3x_prefill.hip - the prefill path of the MoE block (more than 8 tokens per call):
 //
 //   pf_split    activations to bf16 hi/lo rows (the GEMMs' B source); clears the histogram
-//   pf_router   router logits of every (token, expert) in double, one sequential chain per
-//               pair in the reference's order (k3_router, k3_ops.c:1666-1688), so they
-//               are the reference's logits bit for bit; sigmoid, + bias (:1691-1692)
-//   pf_topk     each token's top-k by one wave (:1700-1716) and the per-expert histogram
+//   pf_router   router logits of every (token, expert) in double, with a bound on their
+//               distance from the reference's chain (k3_router, k3_ops.c:1666-1688)
+//   pf_topk     sigmoid, + bias (:1691-1692), each token's top-k by one wave (:1700-1716),
+//               logits that the bound does not prove and that could reach it worked out
+//               again as the chain, so the routing is the reference's bit for bit; and
+//               the per-expert histogram
 //   pf_scan     per-expert offsets (prefix sum) and the GEMM tile lists
 //   pf_scatter  each (token, slot) to its row in its expert's segment
 //   pf_gather   the routed input's planes, rows in that order
@@ -152,115 +154,305 @@ __global__ void __launch_bounds__(PF_NT) pf_gather(const void *x, int x_bf16, in
 }
 
 // ------------------------------------------------------------------ router
-// Logits of every (token, expert) pair in double, each one sequential chain over
-// i = 0 .. H-1 in the reference's order (k3_router, k3_ops.c:1666-1688), on the FP64
-// matrix cores.  v_mfma_f64_16x16x4f64 adds its four k terms to each output one after
-// another, k in lane-group order, each a fused multiply-add (held bitwise against a
-// sequential fma chain on wide-exponent cancelling data); a product of two floats is
-// exact in double, so the chain equals the reference's fma-free loop bit for bit.  A
-// chain cannot be split over k, so the parallelism is the number of 16x16 output tiles:
-// a workgroup takes 48 experts x 64 tokens as twelve waves of one tile each (three waves
-// a SIMD, whose independent chains keep its matrix core fed; 12 tiles per CU at 2048
-// tokens x 384 experts).  K is staged 64 at a time in LDS as float, element k of a chunk
-// at (k % 4) * 16 + k / 4 of its row, so that one 16-byte read gives a lane its operands
-// of four consecutive MFMA steps; the next chunk is fetched into registers during the
-// current one.  Workgroups are dealt expert block fastest, so that with 8 expert blocks
-// each XCD keeps one block's router rows in L2.
-#define RM_E  48
-#define RM_T  64
+// Logits of every (token, expert) pair in double on the FP64 matrix cores, K cut into
+// segments that run side by side, with a bound on how far the reference's logit, one
+// sequential chain over i = 0 .. H-1 (k3_router, k3_ops.c:1666-1688), can lie from each
+// sum.  The float logit is the chain's wherever the bound proves it (float_proven);
+// pf_topk works a pair that it does not prove out again as the chain, where the pair could
+// reach the token's selection.
+//
+// The bound.  A product of two floats is exact in double, so a chain of additions is off
+// the exact sum by at most 2^-53 times the sum of its partial sums' magnitudes.  Over a
+// chunk c of RM_KC elements every partial sum, in whatever order, is at most |S_c| + P_c:
+// S_c the sum before the chunk, P_c = sum |w_i| max |x_i| over it.  So the two sums
+// together are off by at most 2^-53 of sum_c RM_KC (|S_c| + P_c) for the chain (S_c the
+// prefix: the segment's start plus the segment's own sum before c) and the same with the
+// segment's own sums for this kernel: 2^-53 (sum over segments of n_s |start_s| + 128 B_s),
+// B_s = sum_c (|S_c, own| + P_c), kept in float beside the accumulators; the factor
+// 1 + 2^-10 covers the float roundings and the bound's second-order terms, n 2^-126 the
+// products that underflow in P_c.  On N(0, 1) tokens at the K2 shape that leaves about one
+// (token, expert) pair in 3 10^4 unproven, and one token in a few thousand whose selection
+// it could change (about 45 us of the top-k then); a bound of 2^-53 n sum|p|, for any
+// order, leaves fifteen times as many.
+//
+// The split.  A wave holds 32 experts x 16 NTT tokens (2 x NTT tiles of v_mfma_f64_16x16x4)
+// of one segment; its operands come straight from memory, 32 k a step (lane (r, g): row r,
+// k 8g .. 8g+7, element j the k-slot g of MFMA j: the order of a chunk's additions is
+// free), the next step's loads in flight.  A workgroup's four waves hold four segments,
+// summed in LDS; where the tiles are few, gridDim gives each to SG workgroups as well,
+// whose parts pf_topk adds.  Bound by the FP64 matrix cores past a few hundred tokens, by
+// load latency below.  One sequential chain per tile (three waves a SIMD, 48 experts x 64
+// tokens a workgroup) took 229 us at 16 tokens (8 workgroups, the chain's 1792 dependent
+// steps and a load's latency every 64 k), 294 at 301, 302 at 2048 x 384 experts and 774 at
+// 2048 x 896; now 12, 56, 243 and 530, with the top-k 6 -> 14, 8 -> 15, 17 -> 13 and 40 ->
+// 70 us (it adds the parts and works out the sigmoids).
+#define RM_E  32
 #define RM_KC 64
-#define RM_S  (RM_KC + 4)
-#define RM_NT 768
+#define RM_NT 256
+#define RM_NW (RM_NT / WAVE)
+#define RM_SGMAX 8
 
 struct PfRouterArgs {
     const void  *x;
     int          x_bf16;
-    const float *W, *bias;
+    const float *W;
     int          T, H, E;
-    float       *score, *choice;
+    int          sg;                 // workgroups along K
+    // sg == 1: the float logit and how far the chain's float logit can lie from it (0:
+    // proven), [T][E]; else the parts' sums and bounds [sg][T][E]
+    float       *logit, *gap;
+    double      *psum;
+    float       *pbnd;
 };
 
 typedef double f64x4 __attribute__((ext_vector_type(4)));
 
-__global__ void __launch_bounds__(RM_NT) pf_router(PfRouterArgs a)
+// chunks of segment s of S over H
+__device__ __forceinline__ int rm_seg(int s, int S, int H) { return (int)((long)(H / RM_KC) * s / S); }
+
+// The float logit of a sum v and the distance its chain's float logit can lie from it,
+// given bnd = sum n_s |start_s| + 128 sum B_s.  A sum that is not finite met an infinity
+// or a NaN, as the chain does whatever the order: proven.
+__device__ __forceinline__ float rm_gap(double v, float bnd, int H)
 {
-    __shared__ __attribute__((aligned(16))) float lds[2][RM_E + RM_T][RM_S];
-    const int nEB = (a.E + RM_E - 1) / RM_E;
-    const int e0 = (blockIdx.x % nEB) * RM_E, t0 = (blockIdx.x / nEB) * RM_T;
-    const int tid = threadIdx.x, wave = tid / WAVE, r = tid % 16, g = (tid % WAVE) / 16;
-    const int et = wave % 3, tt = wave / 3;          // this wave's expert and token tiles
-    // staging roles: W row tid/16 (48 rows), k 4*(tid%16) .. +3; x (threads below 512) row
-    // tid/8, k 8*(tid%8) .. +7
-    const int wk = 4 * (tid % 16), xk = 8 * (tid % 8);
-    const bool xst = tid < RM_T * 8;
-    f32x4 wv;
-    float xv[8];
-    auto fetch = [&](int k0) AI {
-        const int e = e0 + tid / 16;
-        wv = e < a.E ? *(const f32x4 *)(a.W + (size_t)e * a.H + k0 + wk) : (f32x4){0.f, 0.f, 0.f, 0.f};
-        if (xst) {
-            const int t = t0 + tid / 8;
-            if (t < a.T) load_x8(a.x, a.x_bf16, (size_t)t * a.H + k0 + xk, xv);
-            else
+    const double d = ((double)bnd * (1.0 + 0x1p-10) + fabs(v) * 64.0 + (double)H * 0x1p-126) * 0x1p-53;
+    const float f = (float)v;
+    if (!isfinite(v) || float_proven(v, d)) return 0.0f;
+    const float lo = (float)(v - d), hi = (float)(v + d);
+    const float gap = fmaxf(hi - f, f - lo);
+    return gap == gap ? gap : __builtin_inff();          // a bound that overflowed: unknown
+}
+
+template <int NTT, bool BF>
+__global__ void __launch_bounds__(RM_NT, 3) pf_router(PfRouterArgs a)
+{
+    constexpr int TT = 16 * NTT, NV = 2 * NTT * 4;           // tokens, values a lane
+    constexpr int XL = BF ? 1 : 2;                           // 16-byte loads of 8 activations
+    __shared__ double sd[RM_NW][NV][WAVE];
+    __shared__ float  sb[RM_NW][NV][WAVE];
+    const int nEB = (a.E + RM_E - 1) / RM_E, nTB = (a.T + TT - 1) / TT;
+    const int eb = blockIdx.x % nEB, tb = (blockIdx.x / nEB) % nTB, sg = blockIdx.x / (nEB * nTB);
+    const int e0 = eb * RM_E, t0 = tb * TT;
+    const int wave = wave_id(), lane = threadIdx.x % WAVE, r = lane & 15, g = lane >> 4;
+    const int S = a.sg * RM_NW, s = sg * RM_NW + wave;
+    const int c0 = rm_seg(s, S, a.H), c1 = rm_seg(s + 1, S, a.H);
+    constexpr uint32_t xes = BF ? 2u : 4u;
+    // rows past the experts or the tokens read out of range: zeros
+    const rsrc_t rw = make_rsrc(a.W + (size_t)e0 * a.H, (uint32_t)min(RM_E, a.E - e0) * (uint32_t)a.H * 4u);
+    const rsrc_t rx = make_rsrc((const uint8_t *)a.x + (size_t)t0 * a.H * xes,
+                                (uint32_t)min(TT, a.T - t0) * (uint32_t)a.H * xes);
+    const uint32_t wo = ((uint32_t)r * (uint32_t)a.H + 8u * g) * 4u;
+    const uint32_t xo = ((uint32_t)r * (uint32_t)a.H + 8u * g) * xes;
+    const uint32_t wrow = 16u * (uint32_t)a.H * 4u, xrow = 16u * (uint32_t)a.H * xes;
+
+    u32x4 wv[2][2][2], xv[2][NTT][XL];
+    auto ld = [&](int slot, int k0) AI {
+        const bool on = k0 < c1 * RM_KC;
 #pragma unroll
-                for (int q = 0; q < 8; q++) xv[q] = 0.f;
+        for (int i = 0; i < 2; i++)
+#pragma unroll
+            for (int h = 0; h < 2; h++)
+                wv[slot][i][h] = bload16(rw, on ? wo + i * wrow + (uint32_t)k0 * 4u + 16u * h : K3X_OOB);
+#pragma unroll
+        for (int i = 0; i < NTT; i++)
+#pragma unroll
+            for (int h = 0; h < XL; h++)
+                xv[slot][i][h] = bload16(rx, on ? xo + i * xrow + (uint32_t)k0 * xes + 16u * h : K3X_OOB);
+    };
+    f64x4 acc[2][NTT];
+    float bnd[2][NTT][4], l1[2], mx[NTT];
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int j = 0; j < NTT; j++) {
+            acc[i][j] = (f64x4){0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+            for (int v = 0; v < 4; v++) bnd[i][j][v] = 0.0f;
+        }
+    auto xval = [&](int slot, int i, int j) AI -> float {
+        if (BF) {
+            const uint32_t d = xv[slot][i][0][j >> 1];
+            return (j & 1) ? __uint_as_float(d & 0xFFFF0000u) : __uint_as_float(d << 16);
+        }
+        return __uint_as_float(xv[slot][i][BF ? 0 : j >> 2][j & 3]);
+    };
+    auto use = [&](int slot) AI {
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            float wf[2], xf[NTT];
+#pragma unroll
+            for (int i = 0; i < 2; i++) {
+                wf[i] = __uint_as_float(wv[slot][i][j >> 2][j & 3]);
+                l1[i] += fabsf(wf[i]);
+            }
+#pragma unroll
+            for (int i = 0; i < NTT; i++) {
+                xf[i] = xval(slot, i, j);
+                mx[i] = fmaxf(mx[i], fabsf(xf[i]));
+            }
+#pragma unroll
+            for (int i = 0; i < 2; i++)
+#pragma unroll
+                for (int t = 0; t < NTT; t++)
+                    acc[i][t] = __builtin_amdgcn_mfma_f64_16x16x4f64((double)wf[i], (double)xf[t],
+                                                                     acc[i][t], 0, 0, 0);
         }
     };
-    auto stage = [&](int b) AI {
+    SCHED_FENCE();
+    ld(0, c0 * RM_KC);
+    SCHED_FENCE();
+    ld(1, c0 * RM_KC + 32);
+    SCHED_FENCE();
+    for (int c = c0; c < c1; c++) {
+        // the chunk's start, before its products
 #pragma unroll
-        for (int q = 0; q < 4; q++) lds[b][tid / 16][q * 16 + tid % 16] = wv[q];
-        if (xst)
+        for (int i = 0; i < 2; i++)
 #pragma unroll
-            for (int q = 0; q < 8; q++)
-                lds[b][RM_E + tid / 8][(q % 4) * 16 + xk / 4 + q / 4] = xv[q];
-    };
-    f64x4 acc = {0.0, 0.0, 0.0, 0.0};
-    fetch(0);
-    stage(0);
-    __syncthreads();
-    const int nk = a.H / RM_KC;
-    for (int kc = 0; kc < nk; kc++) {
-        const int b = kc & 1;
-        if (kc + 1 < nk) fetch((kc + 1) * RM_KC);
+            for (int t = 0; t < NTT; t++)
 #pragma unroll
-        for (int j0 = 0; j0 < RM_KC / 4; j0 += 4) {
-            const f32x4 xq = *(const f32x4 *)&lds[b][RM_E + 16 * tt + r][g * 16 + j0];
-            const f32x4 wq = *(const f32x4 *)&lds[b][16 * et + r][g * 16 + j0];
+                for (int v = 0; v < 4; v++) bnd[i][t][v] += fabsf((float)acc[i][t][v]);
 #pragma unroll
-            for (int jj = 0; jj < 4; jj++)
-                acc = __builtin_amdgcn_mfma_f64_16x16x4f64((double)wq[jj], (double)xq[jj], acc, 0, 0, 0);
+        for (int i = 0; i < 2; i++) l1[i] = 0.0f;
+#pragma unroll
+        for (int i = 0; i < NTT; i++) mx[i] = 0.0f;
+        use(0);
+        SCHED_FENCE();
+        ld(0, (c + 1) * RM_KC);
+        SCHED_FENCE();
+        use(1);
+        SCHED_FENCE();
+        ld(1, (c + 1) * RM_KC + 32);
+        SCHED_FENCE();
+        // P_c: row r's sum |w| and token r's max |x| over the four lanes that share them;
+        // value v of a tile is expert g + 4v
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            l1[i] += __shfl_xor(l1[i], 16);
+            l1[i] += __shfl_xor(l1[i], 32);
         }
-        if (kc + 1 < nk) stage(b ^ 1);
-        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < NTT; i++) {
+            mx[i] = fmaxf(mx[i], __shfl_xor(mx[i], 16));
+            mx[i] = fmaxf(mx[i], __shfl_xor(mx[i], 32));
+        }
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const float p = __shfl(l1[i], g + 4 * v);
+#pragma unroll
+                for (int t = 0; t < NTT; t++) bnd[i][t][v] += p * mx[t];
+            }
     }
-    // element i of lane (r, g): expert 16 et + g + 4i, token 16 tt + r
-    const int t = t0 + 16 * tt + r;
-    if (t >= a.T) return;
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const int e = e0 + 16 * et + g + 4 * i;
-        if (e < a.E) {
-            const float sc = sigmoid_ref((float)acc[i]);
-            a.score[(size_t)t * a.E + e] = sc;
-            a.choice[(size_t)t * a.E + e] = sc + a.bias[e];
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int t = 0; t < NTT; t++)
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                sd[wave][(i * NTT + t) * 4 + v][lane] = acc[i][t][v];
+                sb[wave][(i * NTT + t) * 4 + v][lane] = bnd[i][t][v];
+            }
+    __syncthreads();
+    // value v of lane (r, g) of tile (i, t): expert 16i + g + 4v, token 16t + r
+    for (int p = threadIdx.x; p < RM_E * TT; p += RM_NT) {
+        const int el = p % RM_E, tl = p / RM_E, e = e0 + el, t = t0 + tl;
+        if (e >= a.E || t >= a.T) continue;
+        const int sl = ((el >> 4) * NTT + (tl >> 4)) * 4 + ((el & 15) >> 2);
+        const int ln = (el & 3) * 16 + (tl & 15);
+        double sum = 0.0;
+        float b = 0.0f;
+#pragma unroll
+        for (int w = 0; w < RM_NW; w++) {
+            const int sw = sg * RM_NW + w;
+            const float nw = (float)((rm_seg(sw + 1, S, a.H) - rm_seg(sw, S, a.H) + 1) * RM_KC);
+            b += nw * fabsf((float)sum) + 128.0f * sb[w][sl][ln];
+            sum += sd[w][sl][ln];
+        }
+        if (a.sg == 1) {
+            const size_t o = (size_t)t * a.E + e;
+            a.logit[o] = (float)sum;
+            a.gap[o] = rm_gap(sum, b, a.H);
+        } else {
+            const size_t o = ((size_t)sg * a.T + t) * a.E + e;
+            a.psum[o] = sum;
+            a.pbnd[o] = b;
         }
     }
 }
 
 // ------------------------------------------------------------------ top-k
 struct PfTopkArgs {
-    const float *score, *choice;
-    int          T, E, K, renorm;
+    PfRouterArgs r;                      // the router's inputs and its results
+    const float *bias;                   // [E]
+    int          K, renorm;
     float        routed_scale;
     int         *idx;   float *wt;       // [T][K]
     int         *uidx;  float *uwt;      // optional caller copies
     int         *counts;                 // [E] histogram
 };
 
-// One wave per token, TK_W tokens a workgroup.  The per-expert histogram is counted in LDS
-// first and added to the global counts once per workgroup and expert: a device-scope
-// atomic per (token, slot) serialised on the busiest experts' counters (the Zipf chunk's
-// first expert takes every token).
+// The reference's logit of (token t, expert e), one double chain over i = 0 .. H-1
+// (k3_ops.c:1666-1688), by one wave: the lanes form CH_N products a step (exact in double;
+// -0.0, the identity of the sum, past H) in the wave's LDS buffer, the next step's loads in
+// flight, and every lane adds them in order.
+#define CH_N 256
+__device__ double pf_chain(const PfRouterArgs &a, int t, int e, double *buf, int lane)
+{
+    const uint32_t H = (uint32_t)a.H, xes = a.x_bf16 ? 2u : 4u;
+    const rsrc_t rw = make_rsrc(a.W + (size_t)e * H, H * 4u);
+    const rsrc_t rx = make_rsrc((const uint8_t *)a.x + (size_t)t * H * xes, H * xes);
+    u32x4 w;
+    u32x2 x0, x1;
+    auto ld = [&](uint32_t k) AI {
+        const uint32_t el = k + 4u * (uint32_t)lane;
+        w = bload16(rw, el < H ? el * 4u : K3X_OOB);
+        x0 = __builtin_amdgcn_raw_buffer_load_b64(rx, el < H ? el * xes : K3X_OOB, 0, 0);
+        x1 = __builtin_amdgcn_raw_buffer_load_b64(rx, el < H && xes == 4u ? el * 4u + 8u : K3X_OOB, 0, 0);
+    };
+    double s = 0.0;
+    ld(0u);
+    for (uint32_t k = 0; k < H; k += CH_N) {
+        const bool on = k + 4u * (uint32_t)lane < H;          // H is a multiple of 4
+        float xf[4];
+        if (a.x_bf16) {
+            xf[0] = bf2f(x0[0] & 0xFFFFu); xf[1] = bf2f(x0[0] >> 16);
+            xf[2] = bf2f(x0[1] & 0xFFFFu); xf[3] = bf2f(x0[1] >> 16);
+        } else {
+            xf[0] = __uint_as_float(x0[0]); xf[1] = __uint_as_float(x0[1]);
+            xf[2] = __uint_as_float(x1[0]); xf[3] = __uint_as_float(x1[1]);
+        }
+        double p[4];
+#pragma unroll
+        for (int q = 0; q < 4; q++) p[q] = on ? (double)__uint_as_float(w[q]) * (double)xf[q] : -0.0;
+        *(f64x2 *)(buf + 4 * lane) = (f64x2){p[0], p[1]};
+        *(f64x2 *)(buf + 4 * lane + 2) = (f64x2){p[2], p[3]};
+        ld(k + CH_N);
+        // one wave: its LDS operations complete in order
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll 8
+        for (int j = 0; j < CH_N; j += 2) {
+            const f64x2 v = *(const f64x2 *)(buf + j);
+            s += v[0];
+            s += v[1];
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    }
+    return s;
+}
+
+// One wave per token, TK_W tokens a workgroup: the scores and choices from the router's
+// logits, the selection, and, while an expert whose logit is not proven could reach it
+// (slack_reaches: its choice plus its slack is at least the K-th choice; every selected
+// expert's is), those experts' logits as the chain and the selection again.  Every pass
+// proves at least one more expert, so the loop ends; then the selected experts' choices
+// are the reference's and every other one lies below the K-th: the selection and its
+// weights are the reference's.  The per-expert histogram is counted in LDS first and
+// added to the global counts once per workgroup and expert: a device-scope atomic per
+// (token, slot) serialised on the busiest experts' counters (the Zipf chunk's first expert
+// takes every token).
 #define TK_W 8
 template <int NE>
 __global__ void __launch_bounds__(TK_W * WAVE) pf_topk(PfTopkArgs a)
@@ -268,16 +460,106 @@ __global__ void __launch_bounds__(TK_W * WAVE) pf_topk(PfTopkArgs a)
     __shared__ int      s_idx[TK_W][K3X_MAX_TOPK];
     __shared__ float    s_w[TK_W][K3X_MAX_TOPK];
     __shared__ int      hist[1024];
-    const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
+    __shared__ __attribute__((aligned(16))) double chain[TK_W][CH_N];
+    const int wave = wave_id(), lane = threadIdx.x % WAVE;
+    const int T = a.r.T, E = a.r.E, H = a.r.H;
     const int t = blockIdx.x * TK_W + wave;
     if (a.counts)
-        for (int e = threadIdx.x; e < a.E; e += TK_W * WAVE) hist[e] = 0;
+        for (int e = threadIdx.x; e < E; e += TK_W * WAVE) hist[e] = 0;
     __syncthreads();
-    if (t < a.T) {                                       // uniform over the wave
-        const rsrc_t cr = make_rsrc(a.choice, (uint32_t)((size_t)a.T * a.E * 4));
-        const rsrc_t sr = make_rsrc(a.score, (uint32_t)((size_t)a.T * a.E * 4));
-        wave_topk<NE, 0>(cr, sr, (uint32_t)((size_t)t * a.E * 4), a.E, a.K, a.renorm,
-                         a.routed_scale, s_idx[wave], s_w[wave], lane);
+    if (t < T) {                                       // uniform over the wave
+        // range-checked loads (an expert past E reads zeros): a load behind a branch would
+        // be waited for on its own
+        float sc[NE], cv[NE], sl[NE], bi[NE];
+        const uint32_t ro = (uint32_t)(t * E + lane * NE);
+        const rsrc_t rb = make_rsrc(a.bias, (uint32_t)E * 4u);
+#pragma unroll
+        for (int c = 0; c < NE; c++) bi[c] = bload_f32<0>(rb, 4u * (uint32_t)(lane * NE + c));
+        if (a.r.sg == 1) {
+            const rsrc_t rl = make_rsrc(a.r.logit, (uint32_t)(T * E) * 4u);
+            const rsrc_t rg = make_rsrc(a.r.gap, (uint32_t)(T * E) * 4u);
+#pragma unroll
+            for (int c = 0; c < NE; c++) {
+                const uint32_t o = lane * NE + c < E ? 4u * (ro + c) : K3X_OOB;
+                sc[c] = bload_f32<0>(rl, o);
+                sl[c] = bload_f32<0>(rg, o);
+            }
+        } else {
+            const int sg = a.r.sg;
+            const rsrc_t rs = make_rsrc(a.r.psum, (uint32_t)(sg * T * E) * 8u);
+            const rsrc_t rg = make_rsrc(a.r.pbnd, (uint32_t)(sg * T * E) * 4u);
+            double sum[NE];
+            float b[NE];
+#pragma unroll
+            for (int c = 0; c < NE; c++) { sum[c] = 0.0; b[c] = 0.0f; }
+            // two parts' loads in flight (one where the registers hold no more)
+            constexpr int D = NE <= 8 ? 2 : 1;
+            u32x2 v[D][NE];
+            float w[D][NE];
+            auto ld = [&](int i, int g) AI {
+#pragma unroll
+                for (int c = 0; c < NE; c++) {
+                    const uint32_t o = ((g < sg) & (lane * NE + c < E)) ? ro + c + (uint32_t)(g * T * E) : K3X_OOB / 8u;
+                    v[i][c] = __builtin_amdgcn_raw_buffer_load_b64(rs, 8u * o, 0, 0);
+                    w[i][c] = bload_f32<0>(rg, 4u * o);
+                }
+            };
+#pragma unroll
+            for (int i = 0; i < D; i++) {
+                SCHED_FENCE();
+                ld(i, i);
+            }
+            SCHED_FENCE();
+            for (int g0 = 0; g0 < sg; g0 += D) {
+#pragma unroll
+                for (int i = 0; i < D; i++) {
+                    const int g = g0 + i, S = sg * RM_NW;   // a part past the last adds zeros
+                    const float n = (float)((rm_seg((g + 1) * RM_NW, S, H) - rm_seg(g * RM_NW, S, H) + 1) * RM_KC);
+#pragma unroll
+                    for (int c = 0; c < NE; c++) {
+                        b[c] += (g < sg ? n * fabsf((float)sum[c]) : 0.0f) + w[i][c];
+                        sum[c] += __builtin_bit_cast(double, v[i][c]);
+                    }
+                    SCHED_FENCE();
+                    ld(i, g + D);
+                    SCHED_FENCE();
+                }
+            }
+#pragma unroll
+            for (int c = 0; c < NE; c++) {
+                sc[c] = (float)sum[c];
+                sl[c] = rm_gap(sum[c], b[c], H);
+            }
+        }
+#pragma unroll
+        for (int c = 0; c < NE; c++) {
+            sc[c] = sigmoid_ref(sc[c]);
+            cv[c] = sc[c] + bi[c];
+            if (sl[c] != 0.0f) sl[c] = logit_slack(sl[c], bi[c]);
+        }
+        for (;;) {
+            float ck;
+            wave_topk_vals<NE>(cv, sc, E, a.K, a.renorm, a.routed_scale, s_idx[wave], s_w[wave],
+                               lane, nullptr, nullptr, &ck);
+            uint32_t crit = 0u;
+#pragma unroll
+            for (int c = 0; c < NE; c++)
+                if (lane * NE + c < E && sl[c] > 0.0f && slack_reaches(slack_key(cv[c], sl[c]), ck))
+                    crit |= 1u << c;
+            if (__ballot(crit != 0u) == 0ull) break;
+            for (;;) {
+                const uint64_t m = __ballot(crit != 0u);
+                if (m == 0ull) break;
+                const int l0 = (int)__builtin_ctzll(m);
+                const int cc = __builtin_ctz((uint32_t)__builtin_amdgcn_readlane((int)crit, l0));
+                const float f = (float)pf_chain(a.r, t, l0 * NE + cc, chain[wave], lane);
+                const float s = sigmoid_ref(f);
+                if (lane == l0) crit &= crit - 1u;
+#pragma unroll
+                for (int c = 0; c < NE; c++)
+                    if (lane == l0 && c == cc) { sc[c] = s; cv[c] = s + bi[c]; sl[c] = 0.0f; }
+            }
+        }
         __builtin_amdgcn_wave_barrier();
         if (lane < a.K) {
             const size_t o = (size_t)t * a.K + lane;
@@ -290,7 +572,7 @@ __global__ void __launch_bounds__(TK_W * WAVE) pf_topk(PfTopkArgs a)
     }
     if (!a.counts) return;                               // uniform
     __syncthreads();
-    for (int e = threadIdx.x; e < a.E; e += TK_W * WAVE)
+    for (int e = threadIdx.x; e < E; e += TK_W * WAVE)
         if (hist[e]) atomicAdd(&a.counts[e], hist[e]);
 }
 
@@ -1329,7 +1611,7 @@ static inline unsigned cdiv(size_t a, size_t b) { return (unsigned)((a + b - 1) 
 template <int NE>
 static void launch_topk(const PfTopkArgs &a, hipStream_t s)
 {
-    hipLaunchKernelGGL(pf_topk<NE>, dim3(cdiv(a.T, TK_W)), dim3(TK_W * WAVE), 0, s, a);
+    hipLaunchKernelGGL(pf_topk<NE>, dim3(cdiv(a.r.T, TK_W)), dim3(TK_W * WAVE), 0, s, a);
 }
 
 // Launch shapes of the routed GEMMs (pf_gemm32): NW waves of RT32 32-row tiles per
@@ -1415,6 +1697,51 @@ static void launch_dense(const PfGemmArgs &a, int HL, hipStream_t s)
         hipLaunchKernelGGL((pf_dense<NMAT, RW, CW, 2, GU, DENSE_NS>), dim3(grid), dim3(PF_NT), 0, s, a);
 }
 
+template <int NTT>
+static void launch_router(const PfRouterArgs &a, hipStream_t s)
+{
+    const dim3 grid(cdiv(a.E, RM_E) * cdiv(a.T, 16 * NTT) * (unsigned)a.sg);
+    if (a.x_bf16) hipLaunchKernelGGL((pf_router<NTT, true>), grid, dim3(RM_NT), 0, s, a);
+    else          hipLaunchKernelGGL((pf_router<NTT, false>), grid, dim3(RM_NT), 0, s, a);
+}
+
+// Router and top-k of T rows: idx and wt, copies in uidx and uwt, the histogram in counts
+// (cleared before; all three may be NULL).
+static int route_rows(k3x_moe_layer *L, const k3x_prefill_buf *B, const void *x, int x_bf16, int T,
+                      int *idx, float *wt, int *uidx, float *uwt, int *counts, hipStream_t s)
+{
+    const k3x_cfg *c = &L->cfg;
+    const int H = c->hidden, E = c->n_experts, K = c->topk;
+    const int ntt = T <= 16 ? 1 : 2;
+    PfTopkArgs at;
+    PfRouterArgs &ar = at.r;
+    ar.x = x; ar.x_bf16 = x_bf16; ar.W = L->router; ar.T = T; ar.H = H; ar.E = E;
+    // workgroups along K: up to three a CU (the LDS holds three), each wave at least one
+    // chunk; the parts' sums and bounds lie in the routed input's planes, which are written
+    // after the top-k
+    const unsigned tiles = cdiv(E, RM_E) * cdiv(T, 16 * ntt);
+    int sg = tiles < 768u / RM_SGMAX ? RM_SGMAX : (tiles < 768u ? (int)(768u / tiles) : 1);
+    if (sg > H / RM_KC / RM_NW) sg = H / RM_KC / RM_NW;
+    const size_t room = (size_t)T * K * (L->XL > H ? L->XL : H) * 4 / ((size_t)T * E * 12);
+    if ((size_t)sg > room) sg = (int)room;
+    ar.sg = sg < 1 ? 1 : sg;
+    ar.logit = B->logit; ar.gap = B->gap;
+    ar.psum = (double *)B->xp;
+    ar.pbnd = (float *)(ar.psum + (size_t)ar.sg * T * E);
+    if (ntt == 1) launch_router<1>(ar, s);
+    else          launch_router<2>(ar, s);
+    int rc = launch_ok();
+    if (rc) return rc;
+    at.bias = L->bias; at.K = K; at.renorm = c->moe_renorm; at.routed_scale = c->routed_scale;
+    at.idx = idx; at.wt = wt; at.uidx = uidx; at.uwt = uwt; at.counts = counts;
+    if (E <= 128)      launch_topk<2>(at, s);
+    else if (E <= 256) launch_topk<4>(at, s);
+    else if (E <= 384) launch_topk<6>(at, s);
+    else if (E <= 512) launch_topk<8>(at, s);
+    else               launch_topk<16>(at, s);
+    return launch_ok();
+}
+
 static int pf_chunk(k3x_moe_layer *L, const k3x_prefill_buf *B, float *out, const void *x,
                     int x_dtype, int T, const float *resid, int *uidx, float *uwt,
                     hipStream_t s)
@@ -1433,11 +1760,13 @@ static int pf_chunk(k3x_moe_layer *L, const k3x_prefill_buf *B, float *out, cons
     if ((rc = launch_ok())) return rc;
 
     // The shared expert (bf16 weights, every token) needs only the split activations: its
-    // gate/up and down run on the layer's side stream, forked right after the split, beside
-    // the router, the dispatch and the routed GEMMs on s (measured against forking after
-    // the dispatch, after the large experts' gate/up or after all routed gate/up: 3.83
-    // against 3.83, 3.88 and 3.91 ms at 2048 tokens).  Its T rows follow the TK routed rows
-    // in y, which nothing on s writes.
+    // gate/up and down run on the layer's side stream, beside the dispatch and the routed
+    // GEMMs on s.  The library's kernels hold every CU while they run, so that the top-k
+    // behind the router waits for a free one: they are forked after it (3.26 to 3.30 ms at
+    // 2048 tokens against 3.37 to 3.46 forked before the router, 3.28 to 3.33 after
+    // pf_tiles).  pf_dense's, two workgroups a CU, let it in: forked before the router (0.89
+    // ms against 0.93 for a 16-token MoE half, 7.67 against 7.70 at the K3 shape's 2048).
+    // Its T rows follow the TK routed rows in y, which nothing on s writes.
     bool forked = false;
     // The library path (bf16 rows, 2*SI <= H, a kernel for each shape): the gate/up product
     // into fp32 rows [T][2*SI] held in the shared rows of y (nothing else writes them before
@@ -1503,24 +1832,10 @@ static int pf_chunk(k3x_moe_layer *L, const k3x_prefill_buf *B, float *out, cons
     // from the fork on, a failed launch joins the side stream before it returns
 #define PF_RET(e) do { const int e_ = (e); \
         if (forked) (void)hipStreamWaitEvent(s, (hipEvent_t)L->pf_ev[1], 0); return e_; } while (0)
-    if ((rc = fork_shared())) return rc;
 
-    PfRouterArgs ar;
-    ar.x = x; ar.x_bf16 = x_bf16; ar.W = L->router; ar.bias = L->bias;
-    ar.T = T; ar.H = H; ar.E = E; ar.score = B->score; ar.choice = B->choice;
-    hipLaunchKernelGGL(pf_router, dim3(cdiv(T, RM_T) * cdiv(E, RM_E)), dim3(RM_NT), 0, s, ar);
-    if ((rc = launch_ok())) PF_RET(rc);
-
-    PfTopkArgs at;
-    at.score = B->score; at.choice = B->choice; at.T = T; at.E = E; at.K = K;
-    at.renorm = c->moe_renorm; at.routed_scale = c->routed_scale;
-    at.idx = B->idx; at.wt = B->wt; at.uidx = uidx; at.uwt = uwt; at.counts = B->counts;
-    if (E <= 128)      launch_topk<2>(at, s);
-    else if (E <= 256) launch_topk<4>(at, s);
-    else if (E <= 384) launch_topk<6>(at, s);
-    else if (E <= 512) launch_topk<8>(at, s);
-    else               launch_topk<16>(at, s);
-    if ((rc = launch_ok())) PF_RET(rc);
+    if (!sh_blas && (rc = fork_shared())) return rc;
+    if ((rc = route_rows(L, B, x, x_bf16, T, B->idx, B->wt, uidx, uwt, B->counts, s))) PF_RET(rc);
+    if (sh_blas && (rc = fork_shared())) return rc;
 
     PfScanArgs sa;
     sa.counts = B->counts; sa.E = E; sa.offsets = B->offsets; sa.cursor = B->cursor;
@@ -1733,14 +2048,12 @@ extern "C" int k3x_dev_prefill(k3x_moe_layer *L, float *out, const void *x, int 
     return 0;
 }
 
-// The router alone (k3x_moe_route): per chunk, every (token, expert) logit as the
-// reference's chain (pf_router) and each token's top-k into the caller's arrays (pf_topk,
-// no histogram).
+// The router alone (k3x_moe_route): per chunk, pf_router and each token's top-k into the
+// caller's arrays (pf_topk, no histogram).
 extern "C" int k3x_dev_route(k3x_moe_layer *L, int *idx, float *wt, const void *x, int x_dtype,
                              int T, void *stream)
 {
-    const k3x_cfg *c = &L->cfg;
-    const int H = c->hidden, E = c->n_experts, K = c->topk;
+    const int H = L->cfg.hidden, K = L->cfg.topk;
     const size_t es = (x_dtype == K3X_BF16) ? 2 : 4;
     const int chunk = k3x_pf_chunk_tokens(L);
     hipStream_t s = (hipStream_t)stream;
@@ -1748,23 +2061,9 @@ extern "C" int k3x_dev_route(k3x_moe_layer *L, int *idx, float *wt, const void *
     if (rc) return rc;
     for (int t0 = 0; t0 < T; t0 += chunk) {
         const int n = T - t0 < chunk ? T - t0 : chunk;
-        PfRouterArgs ar;
-        ar.x = (const char *)x + (size_t)t0 * H * es; ar.x_bf16 = x_dtype == K3X_BF16;
-        ar.W = L->router; ar.bias = L->bias; ar.T = n; ar.H = H; ar.E = E;
-        ar.score = L->pf.score; ar.choice = L->pf.choice;
-        hipLaunchKernelGGL(pf_router, dim3(cdiv(n, RM_T) * cdiv(E, RM_E)), dim3(RM_NT), 0, s, ar);
-        if ((rc = launch_ok())) return rc;
-        PfTopkArgs at;
-        at.score = L->pf.score; at.choice = L->pf.choice; at.T = n; at.E = E; at.K = K;
-        at.renorm = c->moe_renorm; at.routed_scale = c->routed_scale;
-        at.idx = idx + (size_t)t0 * K; at.wt = wt + (size_t)t0 * K;
-        at.uidx = NULL; at.uwt = NULL; at.counts = NULL;
-        if (E <= 128)      launch_topk<2>(at, s);
-        else if (E <= 256) launch_topk<4>(at, s);
-        else if (E <= 384) launch_topk<6>(at, s);
-        else if (E <= 512) launch_topk<8>(at, s);
-        else               launch_topk<16>(at, s);
-        if ((rc = launch_ok())) return rc;
+        if ((rc = route_rows(L, &L->pf, (const char *)x + (size_t)t0 * H * es, x_dtype == K3X_BF16, n,
+                             idx + (size_t)t0 * K, wt + (size_t)t0 * K, NULL, NULL, NULL, s)))
+            return rc;
     }
     return 0;
 }

@@ -23,6 +23,31 @@ __device__ __forceinline__ float key_choice(uint32_t k)
     return __uint_as_float((k & 0x80000000u) ? (k & 0x7FFFFFFFu) : ~k);
 }
 
+// The choice key (choice_key's order) just above choice + slack: an upper bound of the
+// reference's choice for an expert whose logit is not proven.
+__device__ __forceinline__ uint32_t slack_key(float choice, float slack)
+{
+    const uint32_t k = choice_key((float)((double)choice + (double)slack));
+    return (k != 0u && k < 0xFF800000u) ? k + 1u : k;
+}
+
+// Whether an expert not proven could change a selection whose K-th choice is ck, or one
+// of its weights: its choice may reach ck (hk: the token's largest slack_key, 0 = none).
+// Every selected expert's choice is at least ck, so a selected one not proven counts.
+__device__ __forceinline__ bool slack_reaches(uint32_t hk, float ck)
+{
+    return hk != 0u && hk >= choice_key(ck);
+}
+
+// The slack of a choice whose logit's float can lie df from the one it was worked out from:
+// a bound on the distance of the reference's choice, a quarter of df (the sigmoid's slope is
+// at most 1/4) plus the roundings of the sigmoid and of the bias add (a few units in the
+// last place of |choice| <= 2 + |bias|).
+__device__ __forceinline__ float logit_slack(double df, float bias)
+{
+    return (float)((df * 0.25 + (2.0 + fabs((double)bias)) * 0x1p-21) * 1.01);
+}
+
 __device__ __forceinline__ int lanes_below(uint64_t m)
 {
     return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
