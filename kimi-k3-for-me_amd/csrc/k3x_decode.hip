@@ -776,7 +776,7 @@ __device__ void k1_down(const K1Args &a, float *lds, int rt)
 template <int NE, bool LDSB>
 __global__ void __launch_bounds__(NT1) k1_zdown(K1Args a)
 {
-    __shared__ float lds[(NT1 / WAVE - 1) * 4 * WAVE];
+    __shared__ __attribute__((aligned(16))) float lds[(NT1 / WAVE - 1) * 4 * WAVE];
     if (blockIdx.x == 0) {
         ks_route<NE>(a.ks, *(KSLds *)dyn_lds, true);
         return;
@@ -790,7 +790,7 @@ __global__ void __launch_bounds__(NT1) k1_zdown(K1Args a)
 template <int TM>
 __global__ void __launch_bounds__(NT1) k1_router_bset(K1Args a)
 {
-    __shared__ float lds[(NT1 / WAVE - 1) * 8 * WAVE];
+    __shared__ __attribute__((aligned(16))) float lds[(NT1 / WAVE - 1) * 8 * WAVE];
     __shared__ float s_inv[K3X_DECODE_MAX_T];
     WgTrace tr;
     tr.start(a.trace);
@@ -1075,7 +1075,7 @@ __device__ void k2_gateup_body(const K2Args &a, float *lds, int *s_go_p);
 template <bool EXACT, bool LDSB, int NE>
 __global__ void __launch_bounds__(NT) k2_gateup(K2Args a)
 {
-    __shared__ float lds[(NT / WAVE - 1) * 8 * WAVE];
+    __shared__ __attribute__((aligned(16))) float lds[(NT / WAVE - 1) * 8 * WAVE];
     __shared__ int s_go;
     WgTrace tr;
     tr.start(a.trace);
@@ -1391,7 +1391,7 @@ __device__ __forceinline__ void k3_body(const K3Args &a, f32x4 &d, int wave, int
 template <bool EXACT>
 __global__ void __launch_bounds__(NT3) k3_down(K3Args a)
 {
-    __shared__ float lds[(NT3 / WAVE - 1) * 4 * WAVE];
+    __shared__ __attribute__((aligned(16))) float lds[(NT3 / WAVE - 1) * 4 * WAVE];
     WgTrace tr;
     tr.start(a.trace);
     const int wave = wave_id(), lane = threadIdx.x % WAVE;
@@ -1431,7 +1431,7 @@ __global__ void __launch_bounds__(NT3) k3_down(K3Args a)
 template <bool EXACT>
 __global__ void __launch_bounds__(NT3) k3_down2(K3Args a)
 {
-    __shared__ float lds[(NT3 / WAVE - 1) * 8 * WAVE];
+    __shared__ __attribute__((aligned(16))) float lds[(NT3 / WAVE - 1) * 8 * WAVE];
     const int wave = wave_id(), lane = threadIdx.x % WAVE;
     constexpr int NW = NT3 / WAVE;
     const int NC = 2 * a.T;
@@ -1917,7 +1917,7 @@ __device__ __forceinline__ void k4_fuse_norm(const KNArgs &a, float *agg, double
 template <bool FUSE, bool SHL>
 __global__ void __launch_bounds__(NT3) k4_up(K4Args a)
 {
-    __shared__ float lds[(NT3 / WAVE - 1) * 8 * WAVE];
+    __shared__ __attribute__((aligned(16))) float lds[(NT3 / WAVE - 1) * 8 * WAVE];
     __shared__ double dl[NT3 / WAVE][K3X_DECODE_MAX_T];
     __shared__ float s_inv[K3X_DECODE_MAX_T];
     constexpr int NW = NT3 / WAVE;
@@ -2248,7 +2248,7 @@ struct TrunkArgs {
 
 __global__ void __launch_bounds__(NT1) trunk_gemv(TrunkArgs a)
 {
-    __shared__ float lds[(NT1 / WAVE - 1) * 4 * WAVE];
+    __shared__ __attribute__((aligned(16))) float lds[(NT1 / WAVE - 1) * 4 * WAVE];
     const int rt = blockIdx.x, lane = threadIdx.x % WAVE;
     float acc[4];
     bf16_tile_x(a.W + (size_t)rt * 16 * a.in, a.in, a.x, a.x_bf16, a.ldx, a.T, lds, acc);

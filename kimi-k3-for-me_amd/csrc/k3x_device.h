@@ -86,22 +86,29 @@ __device__ __forceinline__ bool float_proven(double v, double d)
 
 // The reference's chain sum_i (double)(a[i] * s) * (double)b[i] for i = 0 .. n-1 in order
 // (s = 1: sum_i a[i] b[i]; a = b: the sum of squares of k3_ops.c:135-136), worked out by
-// a workgroup of nt threads: chunks of C elements of a and b staged in buf (2C floats of
-// LDS), thread 0 adds them.  Every thread calls; the value in thread 0.  For the rare
-// sums whose float result another order does not prove.
+// a workgroup of nt threads: the products of C elements (exact in double; -0.0, the
+// identity of the sum, past n) staged in buf (2C floats of LDS, 16-byte aligned; C a
+// multiple of 2), thread 0 adds them.  Every thread calls; the value in thread 0.  For the
+// rare sums whose float result another order does not prove.
 __device__ double wg_dot_chain(const float *a, float s, const float *b, int n, float *buf, int C,
                                int nt)
 {
+    double *pl = (double *)buf;
     double acc = 0.0;
     for (int i0 = 0; i0 < n; i0 += C) {
-        const int m = n - i0 < C ? n - i0 : C;
-        for (int i = threadIdx.x; i < m; i += nt) {
-            buf[i] = a[i0 + i];
-            buf[C + i] = b[i0 + i];
-        }
+        for (int i = threadIdx.x; i < C; i += nt)
+            pl[i] = i0 + i < n ? (double)(a[i0 + i] * s) * (double)b[i0 + i] : -0.0;
         __syncthreads();
-        if (threadIdx.x == 0)
-            for (int i = 0; i < m; i++) acc += (double)(buf[i] * s) * (double)buf[C + i];
+        if (threadIdx.x == 0) {
+            double t = acc;
+#pragma unroll 8
+            for (int i = 0; i < C; i += 2) {
+                const f64x2 v = *(const f64x2 *)(pl + i);
+                t += v[0];
+                t += v[1];
+            }
+            acc = t;
+        }
         __syncthreads();
     }
     return acc;

@@ -3,8 +3,12 @@
 // per row as k3_decoder_layer_core takes them, :2481-2493) and a float row copy.
 #include "k3x_device.h"
 
-#define AR_NT 256
+#define AR_NT 1024
+#define AR_NW (AR_NT / WAVE)
 #define AR_MAXSRC 64
+#define AR_U 7                    // float4 loads a lane keeps in flight
+#define AR_CH 1024                // products of a chain chunk
+#define CP_NT 256
 
 __device__ __forceinline__ const float *ar_src(const float *blocks, int maxb, int nb,
                                                const float *pref, int n, int t, int s)
@@ -12,16 +16,74 @@ __device__ __forceinline__ const float *ar_src(const float *blocks, int maxb, in
     return s < nb ? blocks + ((size_t)t * maxb + s) * n : pref + (size_t)t * n;
 }
 
-// Double sum of a per-thread partial over the workgroup (every thread gets it).
-__device__ __forceinline__ double ar_sum(double v, double *red)
+// Sum over the wave of a double (every lane).
+__device__ __forceinline__ double ar_wsum(double v)
 {
-    const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE;
     for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off);
+    return v;
+}
+
+// Elements of half `half` of a row of n floats for this lane: f(j, v, w) for its elements,
+// j counting them (v of row a, w of row b, or of a again with b NULL).  float4 loads (VEC:
+// n a multiple of 4, rows 16-byte aligned), AR_U of each row in flight, zeros past the row.
+template <bool VEC, class F>
+__device__ __forceinline__ void ar_half(const float *a, const float *b, int n, int half, int lane, F f)
+{
+    const int l = half * WAVE + lane;
+    if (!VEC) {
+        int j = 0;
+        for (int i = l; i < n; i += 2 * WAVE, j++) f(j, a[i], b ? b[i] : a[i]);
+        return;
+    }
+    const rsrc_t ra = make_rsrc(a, (uint32_t)n * 4u), rb = make_rsrc(b ? b : a, (uint32_t)n * 4u);
+    for (int f0 = 0; f0 < n; f0 += 8 * WAVE * AR_U) {
+        u32x4 va[AR_U], vb[AR_U];
+#pragma unroll
+        for (int u = 0; u < AR_U; u++) {
+            const uint32_t o = (uint32_t)(f0 + 8 * WAVE * u + 4 * l) * 4u;
+            va[u] = bload16(ra, o);
+            if (b) vb[u] = bload16(rb, o);
+        }
+        SCHED_FENCE();
+#pragma unroll
+        for (int u = 0; u < AR_U; u++)
+#pragma unroll
+            for (int k = 0; k < 4; k++)
+                f(k, __uint_as_float(va[u][k]), __uint_as_float(b ? vb[u][k] : va[u][k]));
+    }
+}
+
+// An upper bound of the sum of the magnitudes of the partial sums S_i of the chain that
+// wg_dot_chain adds (every thread): each thread's run of consecutive products, the runs'
+// sums scanned, then each run's partial sums.  In double; the roundings of this evaluation
+// are covered by the caller's margin.
+__device__ double ar_prefix_mag(const float *a, float s, const float *b, int n, double *wt)
+{
+    const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
+    const int m = (n + AR_NT - 1) / AR_NT, i0 = threadIdx.x * m, i1 = min(n, i0 + m);
+    double run = 0.0;
+    for (int i = i0; i < i1; i++) run += (double)(a[i] * s) * (double)b[i];
+    double in = run;
+    for (int o = 1; o < WAVE; o <<= 1) {
+        const double t = __shfl_up(in, o);
+        if (lane >= o) in += t;
+    }
     __syncthreads();
-    if (lane == 0) red[wave] = v;
+    if (lane == WAVE - 1) wt[wave] = in;
+    __syncthreads();
+    double x = in - run;
+    for (int w = 0; w < wave; w++) x += wt[w];
+    double mag = 0.0;
+    for (int i = i0; i < i1; i++) {
+        x += (double)(a[i] * s) * (double)b[i];
+        mag += fabs(x);
+    }
+    mag = ar_wsum(mag);
+    __syncthreads();
+    if (lane == 0) wt[wave] = mag;
     __syncthreads();
     double tot = 0.0;
-    for (int w = 0; w < AR_NT / WAVE; w++) tot += red[w];
+    for (int w = 0; w < AR_NW; w++) tot += wt[w];
     return tot;
 }
 
@@ -37,70 +99,126 @@ __device__ __forceinline__ double ar_sum(double v, double *red)
 // float, in source order from 0 (the raw rows are the values).  A device count outside
 // 0 .. min(maxb, AR_MAXSRC - 1) (or above 0 without blocks) fills row t with quiet NaNs
 // instead: the reference reads past its stack there.
+//
+// Two waves a source, every source of up to eight at once: bound by the latency of a row's
+// two dependent passes, not by its bytes.  (256 threads walking the sources one after
+// another took 59 us at one row of 6 sources of 7168, 88 at 16 rows, 411 where a key's
+// chain was needed, 827 at 256; now 13, 13 to 20 and 31.)  A key is tested twice: first
+// by chain_gap, which assumes every partial sum as large as sum |p| (about one key in 800
+// of random rows fails), then by the partial sums' own magnitudes (one in 50,000).
+template <bool VEC>
 __global__ void __launch_bounds__(AR_NT) attn_res_kernel(float *h, const float *blocks, int maxb,
                                                          int nb0, const int *nbv, int nbs,
                                                          const float *pref,
                                                          const float *fold, int n, float eps)
 {
-    __shared__ double red[AR_NT / WAVE];
-    __shared__ float p[AR_MAXSRC];
-    __shared__ float sc[AR_MAXSRC];
-    __shared__ float buf[2 * 512];
-    __shared__ double s_ss;
-    const int t = blockIdx.x;
+    __shared__ double red[AR_MAXSRC][2];
+    __shared__ float reda[AR_MAXSRC][2], inv[AR_MAXSRC], p[AR_MAXSRC], sc[AR_MAXSRC];
+    __shared__ int redo[AR_MAXSRC];
+    __shared__ double wt[AR_NW];
+    __shared__ __attribute__((aligned(16))) float buf[2 * AR_CH];
+    const int t = blockIdx.x, wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
     const int nb = nbv ? nbv[(size_t)t * nbs] : nb0;
     if (nb < 0 || nb > maxb || nb + 1 > AR_MAXSRC || (nb > 0 && !blocks)) {
         for (int i = threadIdx.x; i < n; i += AR_NT) h[(size_t)t * n + i] = __int_as_float(0x7FC00000);
         return;
     }
     const int nsrc = nb + 1;
-    for (int s = 0; s < nsrc; s++) {
-        const float *v = ar_src(blocks, maxb, nb, pref, n, t, s);
-        double ss = 0.0;
-        for (int i = threadIdx.x; i < n; i += AR_NT) ss += (double)v[i] * (double)v[i];
-        ss = ar_sum(ss, red);
-        if (!rms_inv_proven(ss, n, eps)) {             // uniform; rare
-            const double c = wg_dot_chain(v, 1.0f, v, n, buf, 512, AR_NT);
-            if (threadIdx.x == 0) s_ss = c;
-            __syncthreads();
-            ss = s_ss;
-        }
-        const float inv = rms_inv(ss, n, eps);
-        double acc = 0.0;
-        float aa = 0.0f;                               // sum |v*inv| |fold|, for the gap
-        for (int i = threadIdx.x; i < n; i += AR_NT) {
-            const float vi = v[i] * inv;
-            acc += (double)vi * (double)fold[i];
-            aa = fmaf(fabsf(vi), fabsf(fold[i]), aa);
-        }
-        acc = ar_sum(acc, red);
-        const double asum = ar_sum((double)aa, red);
-        if (!float_proven(acc, chain_gap(abs_bound((float)asum, n), n)))   // uniform; rare
-            acc = wg_dot_chain(v, inv, fold, n, buf, 512, AR_NT);          // thread 0's
-        if (threadIdx.x == 0) sc[s] = (float)acc;
+    // sums of squares: an element takes part in at most n/512 + 11 additions
+    for (int it = wave; it < 2 * nsrc; it += AR_NW) {
+        double a4[4] = {0.0, 0.0, 0.0, 0.0};
+        ar_half<VEC>(ar_src(blocks, maxb, nb, pref, n, t, it >> 1), nullptr, n, it & 1, lane,
+                     [&](int j, float v, float) AI { a4[j & 3] += (double)v * (double)v; });
+        const double ss = ar_wsum((a4[0] + a4[1]) + (a4[2] + a4[3]));
+        if (lane == 0) red[it >> 1][it & 1] = ss;
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
+    if (threadIdx.x < nsrc) {
+        const double ss = red[threadIdx.x][0] + red[threadIdx.x][1];
+        inv[threadIdx.x] = rms_inv(ss, n, eps);
+        redo[threadIdx.x] = !rms_inv_proven(ss, n, eps);
+    }
+    __syncthreads();
+    for (int s = 0; s < nsrc; s++) {
+        if (!redo[s]) continue;                                          // uniform; rare
+        const float *v = ar_src(blocks, maxb, nb, pref, n, t, s);
+        const double c = wg_dot_chain(v, 1.0f, v, n, buf, AR_CH, AR_NT);
+        if (threadIdx.x == 0) inv[s] = rms_inv(c, n, eps);
+        __syncthreads();
+    }
+    // keys, and sum |v*inv| |fold| for the gap
+    for (int it = wave; it < 2 * nsrc; it += AR_NW) {
+        const float iv = inv[it >> 1];
+        double a4[4] = {0.0, 0.0, 0.0, 0.0};
+        float m4[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+        ar_half<VEC>(ar_src(blocks, maxb, nb, pref, n, t, it >> 1), fold, n, it & 1, lane,
+                     [&](int j, float v, float w) AI {
+                         const float vi = v * iv;
+                         a4[j & 3] += (double)vi * (double)w;
+                         m4[j & 3] = fmaf(fabsf(vi), fabsf(w), m4[j & 3]);
+                     });
+        const double acc = ar_wsum((a4[0] + a4[1]) + (a4[2] + a4[3]));
+        float aa = (m4[0] + m4[1]) + (m4[2] + m4[3]);
+        for (int off = 32; off >= 1; off >>= 1) aa += __shfl_xor(aa, off);
+        if (lane == 0) { red[it >> 1][it & 1] = acc; reda[it >> 1][it & 1] = aa; }
+    }
+    __syncthreads();
+    if (threadIdx.x < nsrc) {
+        const int s = threadIdx.x;
+        const double acc = red[s][0] + red[s][1];
+        sc[s] = (float)acc;
+        redo[s] = !float_proven(acc, chain_gap(abs_bound(reda[s][0] + reda[s][1], n), n));
+    }
+    __syncthreads();
+    for (int s = 0; s < nsrc; s++) {
+        if (!redo[s]) continue;                                          // uniform; rare
+        const float *v = ar_src(blocks, maxb, nb, pref, n, t, s);
+        const double acc = red[s][0] + red[s][1];
+        const double as = abs_bound(reda[s][0] + reda[s][1], n);
+        // the chain is within 2^-53 sum |S_i| of the exact sum, this tree within 2^-53
+        // (n/512 + 11) sum |p| (doubled, for the magnitudes' own roundings)
+        const double d = (ar_prefix_mag(v, inv[s], fold, n, wt) * (1.0 + 0x1p-16) +
+                          2.0 * ((double)(n >> 9) + 16.0) * as) * 0x1p-53;
+        if (float_proven(acc, d)) continue;                              // uniform
+        const double c = wg_dot_chain(v, inv[s], fold, n, buf, AR_CH, AR_NT);   // thread 0's
+        if (threadIdx.x == 0) sc[s] = (float)c;
+        __syncthreads();
+    }
+    if (wave == 0) {
         float m = sc[0];
         for (int s = 1; s < nsrc; s++) m = sc[s] > m ? sc[s] : m;
+        const float e = lane < nsrc ? (float)exp((double)(sc[lane] - m)) : 0.0f;
         double z = 0.0;
-        for (int s = 0; s < nsrc; s++) {
-            sc[s] = (float)exp((double)(sc[s] - m));
-            z += sc[s];
-        }
-        for (int s = 0; s < nsrc; s++) p[s] = (float)(sc[s] / z);
+        for (int s = 0; s < nsrc; s++) z += (double)__shfl(e, s);
+        if (lane < nsrc) p[lane] = (float)((double)e / z);
     }
     __syncthreads();
-    for (int i = threadIdx.x; i < n; i += AR_NT) {
-        float o = 0.0f;
-        for (int s = 0; s < nsrc; s++) o += p[s] * ar_src(blocks, maxb, nb, pref, n, t, s)[i];
-        h[(size_t)t * n + i] = o;
+    if (VEC) {
+        for (int i = 4 * threadIdx.x; i < n; i += 4 * AR_NT) {
+            f32x4 o = {0.f, 0.f, 0.f, 0.f};
+            for (int s0 = 0; s0 < nsrc; s0 += 4) {
+                f32x4 v[4];
+#pragma unroll
+                for (int u = 0; u < 4; u++)
+                    if (s0 + u < nsrc) v[u] = *(const f32x4 *)(ar_src(blocks, maxb, nb, pref, n, t, s0 + u) + i);
+#pragma unroll
+                for (int u = 0; u < 4; u++)
+                    if (s0 + u < nsrc) o += p[s0 + u] * v[u];
+            }
+            *(f32x4 *)(h + (size_t)t * n + i) = o;
+        }
+    } else {
+        for (int i = threadIdx.x; i < n; i += AR_NT) {
+            float o = 0.0f;
+            for (int s = 0; s < nsrc; s++) o += p[s] * ar_src(blocks, maxb, nb, pref, n, t, s)[i];
+            h[(size_t)t * n + i] = o;
+        }
     }
 }
 
-__global__ void __launch_bounds__(AR_NT) copy_f32x4(float *dst, const float *src, size_t n4)
+__global__ void __launch_bounds__(CP_NT) copy_f32x4(float *dst, const float *src, size_t n4)
 {
-    const size_t i = (size_t)blockIdx.x * AR_NT + threadIdx.x;
+    const size_t i = (size_t)blockIdx.x * CP_NT + threadIdx.x;
     if (i < n4) ((f32x4 *)dst)[i] = ((const f32x4 *)src)[i];
 }
 
@@ -111,8 +229,15 @@ extern "C" int k3x_dev_attn_res(float *h, const float *blocks, int maxb, int nb,
                                 float eps, void *stream)
 {
     if (!nbv && nb + 1 > AR_MAXSRC) return K3X_E_SHAPE;
-    hipLaunchKernelGGL(attn_res_kernel, dim3(T), dim3(AR_NT), 0, (hipStream_t)stream, h, blocks,
-                       maxb, nb, nbv, nbs, pref, fold, n, eps);
+    // rows of whole 16-byte pieces, every base aligned (blocks is not read when no row has
+    // any); a row past 2^31 bytes keeps the plain loop
+    const uintptr_t al = (uintptr_t)h | (uintptr_t)blocks | (uintptr_t)pref | (uintptr_t)fold;
+    if (n % 4 == 0 && (al & 15) == 0 && n < (1 << 28))
+        hipLaunchKernelGGL(attn_res_kernel<true>, dim3(T), dim3(AR_NT), 0, (hipStream_t)stream, h,
+                           blocks, maxb, nb, nbv, nbs, pref, fold, n, eps);
+    else
+        hipLaunchKernelGGL(attn_res_kernel<false>, dim3(T), dim3(AR_NT), 0, (hipStream_t)stream, h,
+                           blocks, maxb, nb, nbv, nbs, pref, fold, n, eps);
     return hipGetLastError() == hipSuccess ? 0 : K3X_E_HIP;
 }
 
@@ -121,7 +246,7 @@ extern "C" int k3x_dev_attn_res(float *h, const float *blocks, int maxb, int nb,
 extern "C" int k3x_dev_copy_f32(float *dst, const float *src, size_t n, void *stream)
 {
     const size_t n4 = n / 4;
-    hipLaunchKernelGGL(copy_f32x4, dim3((unsigned)((n4 + AR_NT - 1) / AR_NT)), dim3(AR_NT), 0,
+    hipLaunchKernelGGL(copy_f32x4, dim3((unsigned)((n4 + CP_NT - 1) / CP_NT)), dim3(CP_NT), 0,
                        (hipStream_t)stream, dst, src, n4);
     return hipGetLastError() == hipSuccess ? 0 : K3X_E_HIP;
 }

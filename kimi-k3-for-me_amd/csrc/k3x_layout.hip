@@ -174,7 +174,7 @@ __global__ void __launch_bounds__(NT) rmsnorm_kernel(float *y, const float *x, c
                                                       int n, float eps)
 {
     __shared__ double red[NT / WAVE];
-    __shared__ float buf[2 * 512];
+    __shared__ __attribute__((aligned(16))) float buf[2 * 512];
     __shared__ double s_ss;
     const float *xr = x + (size_t)blockIdx.x * n;
     float *yr = y + (size_t)blockIdx.x * n;
