@@ -968,7 +968,8 @@ size_t k3x_pf_layout(const k3x_moe_layer *L, int T, char *p, k3x_prefill_buf *B)
         t * E * 4, t * E * 4,      /* logit, gap */
         t * K * 4, t * K * 4,      /* idx, wt */
         E * 4, (E + 1) * 4, E * 4, /* counts, offsets, cursor */
-        2 * (E + 1) * 4, 2 * (E + 1) * 4,  /* tb_gu, tb_dn: small and large tile classes */
+        2 * (E + 1) * 4, 2 * (E + 1) * 4,  /* tb_gu, tb_dn: E + 6 words (256 bytes hold
+                                              those of E < 4) */
         t * K * 4, t * K * 4, t * K * 4,   /* perm_tok, perm_w, pos_of */
         t * K * I * 4,             /* act     */
         (SI ? t * SI * 4 : 256),   /* act_sh  */

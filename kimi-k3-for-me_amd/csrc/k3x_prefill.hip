@@ -578,39 +578,49 @@ __global__ void __launch_bounds__(TK_W * WAVE) pf_topk(PfTopkArgs a)
 
 // ------------------------------------------------------------------ scan
 // One workgroup of 1024 threads (E <= 1024): offsets[e] = sum of counts below e, and the
-// tile bases of the two routed GEMMs.  Each GEMM has two tile classes: an expert with at
-// most tpb_s tokens takes nrb_s tiles of tpb_s columns (one column block), a larger one
-// nrb_b x ceil(count/tpb_b) tiles of tpb_b columns.  tb[0..E] are the small class's bases
-// (tb[E] = its tile count), tb[E+1 .. 2E+1] the large class's.  Cursors cleared.  Five
-// inclusive scans, one element per thread (shuffles within each wave, then the waves'
-// totals).
+// tile bases of the two routed GEMMs.  Each GEMM has PF_NC tile classes by an expert's
+// tokens: of at most tpb[0], of at most tpb[1] (empty when that is tpb[0]), and the others;
+// class c takes nrb[c] x ceil(count / tpb[c]) tiles of tpb[c] columns.  tb[e] is the first
+// tile of expert e in the GEMM's list (class 0's tiles first, then class 1's, then class
+// 2's); tb[E + 2c] and tb[E + 2c + 1] are class c's number of tiles and its first.  Cursors
+// cleared.  1 + 2 PF_NC inclusive scans, one element per thread (shuffles within each wave,
+// then the waves' totals).
+#define PF_NC 3
+#define PF_NSC (1 + 2 * PF_NC)
+
 struct PfScanArgs {
     const int *counts;
     int        E;
     int       *offsets, *cursor;
     int       *tb[2];                   // gate/up, down
-    int        tpb_s[2], tpb_b[2];      // columns of a tile, small and large class
-    int        nrb_s[2], nrb_b[2];      // row blocks, small and large class
+    int        tpb[2][PF_NC];           // columns of a tile
+    int        nrb[2][PF_NC];           // row blocks
 };
+
+__device__ __forceinline__ int pf_class(const PfScanArgs &a, int m, int c)
+{
+    return c <= a.tpb[m][0] ? 0 : (c <= a.tpb[m][1] ? 1 : 2);
+}
 
 __global__ void __launch_bounds__(1024) pf_scan(PfScanArgs a)
 {
-    __shared__ int wsum[5][16], woff[5][16];
+    __shared__ int wsum[PF_NSC][16], woff[PF_NSC][16], tot[PF_NSC];
     const int e = threadIdx.x, E = a.E, wave = e / WAVE, lane = e % WAVE;
     const int c = e < E ? a.counts[e] : 0;
-    int v[5];
+    int v[PF_NSC];
     v[0] = c;
 #pragma unroll
     for (int m = 0; m < 2; m++) {
-        const bool big = c > a.tpb_s[m];
-        v[1 + 2 * m] = big ? 0 : a.nrb_s[m] * ((c + a.tpb_s[m] - 1) / a.tpb_s[m]);
-        v[2 + 2 * m] = big ? a.nrb_b[m] * ((c + a.tpb_b[m] - 1) / a.tpb_b[m]) : 0;
+        const int k = pf_class(a, m, c);
+#pragma unroll
+        for (int q = 0; q < PF_NC; q++)
+            v[1 + PF_NC * m + q] = k == q ? a.nrb[m][q] * ((c + a.tpb[m][q] - 1) / a.tpb[m][q]) : 0;
     }
     if (e < E) a.cursor[e] = 0;
     // inclusive sums: within each wave by shuffles, then the waves' totals (wave 0)
-    int in[5];
+    int in[PF_NSC];
 #pragma unroll
-    for (int i = 0; i < 5; i++) {
+    for (int i = 0; i < PF_NSC; i++) {
         in[i] = v[i];
 #pragma unroll
         for (int o = 1; o < WAVE; o <<= 1) {
@@ -622,7 +632,7 @@ __global__ void __launch_bounds__(1024) pf_scan(PfScanArgs a)
     __syncthreads();
     if (wave == 0 && lane < 16) {
 #pragma unroll
-        for (int i = 0; i < 5; i++) {
+        for (int i = 0; i < PF_NSC; i++) {
             int x = wsum[i][lane], inc = x;
 #pragma unroll
             for (int o = 1; o < 16; o <<= 1) {
@@ -630,26 +640,37 @@ __global__ void __launch_bounds__(1024) pf_scan(PfScanArgs a)
                 if (lane >= o) inc += t;
             }
             woff[i][lane] = inc - x;
+            if (lane == 15) tot[i] = inc;
         }
     }
     __syncthreads();
 #pragma unroll
-    for (int i = 0; i < 5; i++) in[i] += woff[i][wave];
+    for (int i = 0; i < PF_NSC; i++) in[i] += woff[i][wave];
     // the exclusive value of e is its inclusive sum less its own
     if (e < E) {
         a.offsets[e] = in[0] - v[0];
 #pragma unroll
         for (int m = 0; m < 2; m++) {
-            a.tb[m][e] = in[1 + 2 * m] - v[1 + 2 * m];
-            a.tb[m][E + 1 + e] = in[2 + 2 * m] - v[2 + 2 * m];
+            const int k = pf_class(a, m, c);
+            int base = 0;
+#pragma unroll
+            for (int q = 0; q < PF_NC; q++) {
+                if (k == q) a.tb[m][e] = base + in[1 + PF_NC * m + q] - v[1 + PF_NC * m + q];
+                base += tot[1 + PF_NC * m + q];
+            }
         }
     }
-    if (e == E - 1) {
-        a.offsets[E] = in[0];
+    if (e == 0) {
+        a.offsets[E] = tot[0];
 #pragma unroll
         for (int m = 0; m < 2; m++) {
-            a.tb[m][E] = in[1 + 2 * m];
-            a.tb[m][2 * E + 1] = in[2 + 2 * m];
+            int base = 0;
+#pragma unroll
+            for (int q = 0; q < PF_NC; q++) {
+                a.tb[m][E + 2 * q] = tot[1 + PF_NC * m + q];
+                a.tb[m][E + 2 * q + 1] = base;
+                base += tot[1 + PF_NC * m + q];
+            }
         }
     }
 }
@@ -682,17 +703,14 @@ __global__ void __launch_bounds__(PF_NT) pf_scatter(const int *idx, const float 
 
 // ------------------------------------------------------------------ tile tables
 // One descriptor per GEMM tile: {group, row block, first permuted row, tokens}; expert e
-// owns tiles tb[e] .. of its class's list (the small class's list first, then the large
-// class's from desc + tb[E]), row blocks outer, column blocks inner.
+// owns tiles tb[e] .. of the GEMM's list, row blocks outer, column blocks inner.
 __global__ void __launch_bounds__(PF_NT) pf_tiles(const int *counts, const int *offsets,
                                                   PfScanArgs a, int4 *desc_gu, int4 *desc_dn)
 {
-    const int e = blockIdx.x, c = counts[e], off = offsets[e], E = a.E;
+    const int e = blockIdx.x, c = counts[e], off = offsets[e];
     for (int m = 0; m < 2; m++) {
-        const bool big = c > a.tpb_s[m];
-        const int tpb = big ? a.tpb_b[m] : a.tpb_s[m], nrb = big ? a.nrb_b[m] : a.nrb_s[m];
-        const int *tb = a.tb[m];
-        int4 *desc = (m ? desc_dn : desc_gu) + (big ? tb[E] + tb[E + 1 + e] : tb[e]);
+        const int k = pf_class(a, m, c), tpb = a.tpb[m][k], nrb = a.nrb[m][k];
+        int4 *desc = (m ? desc_dn : desc_gu) + a.tb[m][e];
         const int nc = (c + tpb - 1) / tpb;
         for (int rel = threadIdx.x; rel < nrb * nc; rel += PF_NT) {
             const int rb = rel / nc, cb = rel % nc;
@@ -952,8 +970,8 @@ __global__ void __launch_bounds__(PF_NT) pf_dense(PfGemmArgs a)
 // 32-63).  The B block in LDS is laid out to match: entry ((g*4 + d)*2 + h)*NCOL + col
 // holds those 8 k of column col.  Every product of the quad is formed exactly once;
 // only the order of the fp32 additions differs from the 16x16 form.
-template <bool EXACT, int NMAT, int RT32, int CT32, int HL, bool GU, int NW>
-__global__ void __launch_bounds__(NW * WAVE) pf_gemm32(PfGemmArgs a)
+template <bool EXACT, int NMAT, int RT32, int CT32, int HL, bool GU, int NW, int MINW>
+__global__ void __launch_bounds__(NW * WAVE, MINW) pf_gemm32(PfGemmArgs a)
 {
     constexpr int NTH = NW * WAVE;
     constexpr int NCOL = CT32 * 32;
@@ -1614,53 +1632,54 @@ static void launch_topk(const PfTopkArgs &a, hipStream_t s)
     hipLaunchKernelGGL(pf_topk<NE>, dim3(cdiv(a.r.T, TK_W)), dim3(TK_W * WAVE), 0, s, a);
 }
 
-// Launch shapes of the routed GEMMs (pf_gemm32): NW waves of RT32 32-row tiles per
-// workgroup and CT32 32-column tiles; a small shape for experts of at most one small
-// column block of tokens (little padding, more workgroups per CU) and a large one for the
-// others (fewer re-reads of their weights and activations).
-#define NW_GS     4
-#define NW_DS     4
-#define NW_B      8
-#define GU_RT32   1
-#define GU_RT32_S 2
-#define GU_CT32_S 1
-#define GU_CT32_B 3
-#define DN_RT32   2
-#define DN_RT32_S 2
-#define DN_CT32_S 2
-#define DN_CT32_B 3
-// The small class of a gate/up over hi and lo columns (fp32 input, or z in the latent
-// form): 32 tokens in two column tiles, eight waves of one 32-row tile (256 rows).  With
-// the single 16-token column tile of the bf16 shape, the K3 chunk's experts of 17 to 32
-// tokens (656 of 896) fell to the large class, one 96-KB-LDS workgroup a CU: 8.07 to 8.13
-// ms per chunk now against 8.39 to 8.49 (four waves of 128 rows: the same; four waves of
-// 256 rows, one wave a SIMD: 8.57 to 8.64).
-#ifndef NW_GS2
-#define NW_GS2    8
+// Launch shapes of the routed GEMMs (pf_gemm32): NW waves of RT 32-row tiles per workgroup
+// and CT 32-column tiles, by class.  Class 0 holds the experts of one narrow column tile,
+// class 1 those of two, class 2 the others (wide tiles: fewer re-reads of their weights and
+// activations).  A gate/up of bf16 rows (one column a token) has no class 1: its single
+// column tile holds 32 tokens.  Class 0 of the two-column products is for the small calls,
+// whose experts have a few tokens each: with two column tiles for them half the matrix
+// work, half the LDS reads and, at 64 KB of LDS, a third of the waves a CU were lost (the
+// gate/up of 40 fp32 tokens 520 -> 400 us, of 130 latent ones 1919 -> 1380).
+struct PfShape { int nw, rt, ct, minw; };
+#ifndef S_GU1_0
+#define S_GU1_0 4, 2, 1, 2
 #endif
-#ifndef GU_RT32_S2
-#define GU_RT32_S2 1
+#ifndef S_GU2_0
+#define S_GU2_0 4, 1, 1, 3
 #endif
-#ifndef GU_CT32_S2
-#define GU_CT32_S2 2
+#ifndef S_GU2_1
+#define S_GU2_1 8, 1, 2, 2
 #endif
+#ifndef S_DN_0
+#define S_DN_0 4, 2, 1, 3
+#endif
+#ifndef S_DN_1
+#define S_DN_1 4, 2, 2, 2
+#endif
+static constexpr PfShape GU1[PF_NC] = {{S_GU1_0}, {S_GU1_0}, {8, 1, 3, 2}};   // bf16 rows
+static constexpr PfShape GU2[PF_NC] = {{S_GU2_0}, {S_GU2_1}, {8, 1, 3, 2}};   // hi and lo columns
+static constexpr PfShape DN[PF_NC] = {{S_DN_0}, {S_DN_1}, {8, 2, 3, 2}};
 
-template <bool EXACT, int HL, int CT32, int NW, int RT32 = GU_RT32>
+template <bool EXACT, int HL, int C>
 static void launch_gu(const PfGemmArgs &a, unsigned grid, hipStream_t s)
 {
-    hipLaunchKernelGGL((pf_gemm32<EXACT, 2, RT32, CT32, HL, true, NW>), dim3(grid),
-                       dim3(NW * WAVE), 0, s, a);
+    constexpr PfShape p = HL == 1 ? GU1[C] : GU2[C];
+    hipLaunchKernelGGL((pf_gemm32<EXACT, 2, p.rt, p.ct, HL, true, p.nw, p.minw>), dim3(grid),
+                       dim3(p.nw * WAVE), 0, s, a);
 }
 
-template <bool EXACT, int CT32, int NW, int RT32 = DN_RT32>
+template <bool EXACT, int C>
 static void launch_dn(const PfGemmArgs &a, unsigned grid, hipStream_t s)
 {
-    hipLaunchKernelGGL((pf_gemm32<EXACT, 1, RT32, CT32, 2, false, NW>), dim3(grid),
-                       dim3(NW * WAVE), 0, s, a);
+    constexpr PfShape p = DN[C];
+    hipLaunchKernelGGL((pf_gemm32<EXACT, 1, p.rt, p.ct, 2, false, p.nw, p.minw>), dim3(grid),
+                       dim3(p.nw * WAVE), 0, s, a);
 }
 
 // MXFP8 mode tiles: small class 32 tokens, large class 64; four waves a workgroup, gate/up
 // 128 rows (one 32-row tile a wave), down 256 (two)
+#define MX_GU_RT32 1
+#define MX_DN_RT32 2
 #define MX_CT_S 1
 #define MX_CT_B 2
 #define MX_NW   4
@@ -1696,6 +1715,11 @@ static void launch_dense(const PfGemmArgs &a, int HL, hipStream_t s)
     else
         hipLaunchKernelGGL((pf_dense<NMAT, RW, CW, 2, GU, DENSE_NS>), dim3(grid), dim3(PF_NT), 0, s, a);
 }
+
+// tokens per expert on average from which class 2's products are the longer part
+#ifndef PF_BIG_ROWS
+#define PF_BIG_ROWS 20
+#endif
 
 template <int NTT>
 static void launch_router(const PfRouterArgs &a, hipStream_t s)
@@ -1841,15 +1865,17 @@ static int pf_chunk(k3x_moe_layer *L, const k3x_prefill_buf *B, float *out, cons
     sa.counts = B->counts; sa.E = E; sa.offsets = B->offsets; sa.cursor = B->cursor;
     sa.tb[0] = B->tb_gu; sa.tb[1] = B->tb_dn;
     const bool mx = L->pf_mode == K3X_PREFILL_MXFP8;
-    sa.tpb_s[0] = mx ? MX_CT_S * 32 : (HLr == 1 ? GU_CT32_S : GU_CT32_S2) * 32 / HLr;
-    sa.tpb_b[0] = mx ? MX_CT_B * 32 : GU_CT32_B * 32 / HLr;
-    sa.nrb_s[0] = cdiv(I, mx ? MX_NW * MX_GU_RT32_S * 32
-                             : (HLr == 1 ? NW_GS * GU_RT32_S : NW_GS2 * GU_RT32_S2) * 32);
-    sa.nrb_b[0] = cdiv(I, (mx ? MX_NW : NW_B) * GU_RT32 * 32);
-    sa.tpb_s[1] = mx ? MX_CT_S * 32 : DN_CT32_S * 32 / 2;
-    sa.tpb_b[1] = mx ? MX_CT_B * 32 : DN_CT32_B * 32 / 2;
-    sa.nrb_s[1] = cdiv(X, mx ? MX_NW * MX_DN_RT32_S * 32 : NW_DS * DN_RT32_S * 32);
-    sa.nrb_b[1] = cdiv(X, (mx ? MX_NW : NW_B) * DN_RT32 * 32);
+    const PfShape mgu[PF_NC] = {{MX_NW, MX_GU_RT32_S, MX_CT_S, 0}, {MX_NW, MX_GU_RT32_S, MX_CT_S, 0},
+                                {MX_NW, MX_GU_RT32, MX_CT_B, 0}};
+    const PfShape mdn[PF_NC] = {{MX_NW, MX_DN_RT32_S, MX_CT_S, 0}, {MX_NW, MX_DN_RT32_S, MX_CT_S, 0},
+                                {MX_NW, MX_DN_RT32, MX_CT_B, 0}};
+    const PfShape *shp[2] = {mx ? mgu : (HLr == 1 ? GU1 : GU2), mx ? mdn : DN};
+    for (int q = 0; q < PF_NC; q++)
+        for (int m = 0; m < 2; m++) {
+            const PfShape &p = shp[m][q];
+            sa.tpb[m][q] = p.ct * 32 / (mx ? 1 : (m ? 2 : HLr));
+            sa.nrb[m][q] = cdiv(m ? X : I, p.nw * p.rt * 32);
+        }
     hipLaunchKernelGGL(pf_scan, dim3(1), dim3(1024), 0, s, sa);
     if ((rc = launch_ok())) PF_RET(rc);
     hipLaunchKernelGGL(pf_scatter, dim3(cdiv(TK, PF_NT)), dim3(PF_NT), 0, s, B->idx, B->wt, TK, K,
@@ -1892,15 +1918,20 @@ static int pf_chunk(k3x_moe_layer *L, const k3x_prefill_buf *B, float *out, cons
     }
     if ((rc = launch_ok())) PF_RET(rc);
 
-    // grids: upper bounds of each list (a small expert has one column block; large ones
-    // number at most TK / (tpb_s + 1)); surplus workgroups leave at once
-    unsigned grid_s[2], grid_b[2];
+    // grids: upper bounds of each class (an expert of class 0 or 1 has one column block;
+    // at most TK / (t + 1) experts have more than t tokens); surplus workgroups leave at
+    // once
+    unsigned grid[2][PF_NC];
     for (int m = 0; m < 2; m++) {
-        const size_t nbig = (size_t)TK / (sa.tpb_s[m] + 1);
-        grid_s[m] = round8((size_t)sa.nrb_s[m] * E);
-        grid_b[m] = round8((size_t)sa.nrb_b[m] * (cdiv(TK, sa.tpb_b[m]) + (nbig < (size_t)E ? nbig : (size_t)E)));
+        const size_t ne = E < TK ? E : TK;
+        size_t n[PF_NC] = {ne, (size_t)TK / (sa.tpb[m][0] + 1), (size_t)TK / (sa.tpb[m][1] + 1)};
+        for (int q = 1; q < PF_NC; q++) n[q] = n[q] < ne ? n[q] : ne;
+        if (sa.tpb[m][1] == sa.tpb[m][0]) n[1] = 0;
+        n[2] = n[2] ? n[2] + cdiv(TK, sa.tpb[m][2]) : 0;
+        for (int q = 0; q < PF_NC; q++) grid[m][q] = round8(sa.nrb[m][q] * n[q]);
     }
-    if (grid_s[0] + grid_b[0] > (unsigned)B->ndesc_gu || grid_s[1] + grid_b[1] > (unsigned)B->ndesc_dn)
+    if (grid[0][0] + grid[0][1] + grid[0][2] > (unsigned)B->ndesc_gu ||
+        grid[1][0] + grid[1][1] + grid[1][2] > (unsigned)B->ndesc_dn)
         PF_RET(K3X_E_SHAPE);
 
     // routed gate/up: B rows are the permuted activation rows
@@ -1916,33 +1947,6 @@ static int pf_chunk(k3x_moe_layer *L, const k3x_prefill_buf *B, float *out, cons
     if (mx) {
         g.b8 = xq8; g.b8s = (const uint32_t *)xs8; g.o8 = aq8; g.o8s = as8;
     }
-    PfGemmArgs gb = g;
-    g.ntile = B->tb_gu + E;
-    gb.ntile = B->tb_gu + 2 * E + 1; gb.dbase = B->tb_gu + E;
-    // the large-expert tiles on s.  In the exact mode the small ones run on the side
-    // stream after the shared expert (forked here, after the routed input is written),
-    // beside the large ones, and join before the combine: 3.56 to 3.58 against 3.61 ms
-    // per 2048-token chunk; the MXFP8 products measured slower that way (2.92 against
-    // 2.80 ms) and stay on s.
-    hipStream_t ss = s;
-    const bool split = forked && !mx;
-    if (split) {
-        if (hipEventRecord((hipEvent_t)L->pf_ev[0], s) != hipSuccess ||
-            hipStreamWaitEvent((hipStream_t)L->pf_side, (hipEvent_t)L->pf_ev[0], 0) != hipSuccess)
-            PF_RET(K3X_E_HIP);
-        ss = (hipStream_t)L->pf_side;
-    }
-    if (mx) {
-        hipLaunchKernelGGL((pf_gemm_mx<2, GU_RT32, MX_CT_B, true, MX_NW>), dim3(grid_b[0]), dim3(MX_NW * WAVE), 0, s, gb);
-    } else if (ex_gu) {
-        if (HLr == 1) launch_gu<true, 1, GU_CT32_B, NW_B>(gb, grid_b[0], s);
-        else          launch_gu<true, 2, GU_CT32_B, NW_B>(gb, grid_b[0], s);
-    } else {
-        if (HLr == 1) launch_gu<false, 1, GU_CT32_B, NW_B>(gb, grid_b[0], s);
-        else          launch_gu<false, 2, GU_CT32_B, NW_B>(gb, grid_b[0], s);
-    }
-    if ((rc = launch_ok())) PF_RET(rc);
-
     // routed down: B rows are the activation rows, in permuted order
     PfGemmArgs d;
     memset(&d, 0, sizeof d);
@@ -1951,33 +1955,67 @@ static int pf_chunk(k3x_moe_layer *L, const k3x_prefill_buf *B, float *out, cons
     d.bsrc = B->act; d.brows = TK; d.perm = NULL; d.row_base = 0;
     d.y = B->y; d.out_base = 0;
     if (mx) { d.b8 = aq8; d.b8s = (const uint32_t *)as8; }
-    PfGemmArgs db = d;
-    d.ntile = B->tb_dn + E;
-    db.ntile = B->tb_dn + 2 * E + 1; db.dbase = B->tb_dn + E;
-    if (mx) {
-        hipLaunchKernelGGL((pf_gemm_mx<2, MX_GU_RT32_S, MX_CT_S, true, MX_NW>), dim3(grid_s[0]), dim3(MX_NW * WAVE), 0, ss, g);
-    } else if (ex_gu) {
-        if (HLr == 1) launch_gu<true, 1, GU_CT32_S, NW_GS, GU_RT32_S>(g, grid_s[0], ss);
-        else          launch_gu<true, 2, GU_CT32_S2, NW_GS2, GU_RT32_S2>(g, grid_s[0], ss);
-    } else {
-        if (HLr == 1) launch_gu<false, 1, GU_CT32_S, NW_GS, GU_RT32_S>(g, grid_s[0], ss);
-        else          launch_gu<false, 2, GU_CT32_S2, NW_GS2, GU_RT32_S2>(g, grid_s[0], ss);
+    const bool ex_dn = (L->special & 4) != 0;
+    // class q's tiles of the gate/up (m = 0) or the down GEMM on stream st
+    auto gemm = [&](int m, int q, hipStream_t st) -> int {
+        const unsigned gr = grid[m][q];
+        if (!gr) return 0;
+        PfGemmArgs &p = m ? d : g;
+        p.ntile = (m ? B->tb_dn : B->tb_gu) + E + 2 * q;
+        p.dbase = p.ntile + 1;
+        if (mx && !m) {
+            if (q == 2) hipLaunchKernelGGL((pf_gemm_mx<2, MX_GU_RT32, MX_CT_B, true, MX_NW>), dim3(gr), dim3(MX_NW * WAVE), 0, st, p);
+            else        hipLaunchKernelGGL((pf_gemm_mx<2, MX_GU_RT32_S, MX_CT_S, true, MX_NW>), dim3(gr), dim3(MX_NW * WAVE), 0, st, p);
+        } else if (mx) {
+            if (q == 2) hipLaunchKernelGGL((pf_gemm_mx<1, MX_DN_RT32, MX_CT_B, false, MX_NW>), dim3(gr), dim3(MX_NW * WAVE), 0, st, p);
+            else        hipLaunchKernelGGL((pf_gemm_mx<1, MX_DN_RT32_S, MX_CT_S, false, MX_NW>), dim3(gr), dim3(MX_NW * WAVE), 0, st, p);
+        } else if (m) {
+            if (q == 0)      ex_dn ? launch_dn<true, 0>(p, gr, st) : launch_dn<false, 0>(p, gr, st);
+            else if (q == 1) ex_dn ? launch_dn<true, 1>(p, gr, st) : launch_dn<false, 1>(p, gr, st);
+            else             ex_dn ? launch_dn<true, 2>(p, gr, st) : launch_dn<false, 2>(p, gr, st);
+        } else if (HLr == 1) {
+            if (q != 2) ex_gu ? launch_gu<true, 1, 0>(p, gr, st) : launch_gu<false, 1, 0>(p, gr, st);
+            else        ex_gu ? launch_gu<true, 1, 2>(p, gr, st) : launch_gu<false, 1, 2>(p, gr, st);
+        } else {
+            if (q == 0)      ex_gu ? launch_gu<true, 2, 0>(p, gr, st) : launch_gu<false, 2, 0>(p, gr, st);
+            else if (q == 1) ex_gu ? launch_gu<true, 2, 1>(p, gr, st) : launch_gu<false, 2, 1>(p, gr, st);
+            else             ex_gu ? launch_gu<true, 2, 2>(p, gr, st) : launch_gu<false, 2, 2>(p, gr, st);
+        }
+        return launch_ok();
+    };
+    // In the exact mode the products of classes 0 and 1 and those of class 2 run on two
+    // streams, s and the layer's side stream (forked here, after the routed input is
+    // written; joined before the combine): 3.56 to 3.58 against 3.61 ms per 2048-token
+    // chunk.  The longer of the two goes on s, at once; the other one on the side stream,
+    // after the shared expert.  The MXFP8 products measured slower that way (2.92 against
+    // 2.80 ms) and stay on s.
+    const bool split = forked && !mx;
+    const bool big_first = TK >= PF_BIG_ROWS * E;
+    hipStream_t st[2] = {s, s};                          // classes 0 and 1, class 2
+    if (split) {
+        if (hipEventRecord((hipEvent_t)L->pf_ev[0], s) != hipSuccess ||
+            hipStreamWaitEvent((hipStream_t)L->pf_side, (hipEvent_t)L->pf_ev[0], 0) != hipSuccess)
+            PF_RET(K3X_E_HIP);
+        st[big_first ? 0 : 1] = (hipStream_t)L->pf_side;
     }
-    rc = launch_ok();
-    if (!rc) {
-        if (mx) hipLaunchKernelGGL((pf_gemm_mx<1, MX_DN_RT32_S, MX_CT_S, false, MX_NW>), dim3(grid_s[1]), dim3(MX_NW * WAVE), 0, ss, d);
-        else if (L->special & 4) launch_dn<true, DN_CT32_S, NW_DS, DN_RT32_S>(d, grid_s[1], ss);
-        else                     launch_dn<false, DN_CT32_S, NW_DS, DN_RT32_S>(d, grid_s[1], ss);
-        rc = launch_ok();
+    // issued longest first, gate/up before the down that reads it; on one stream every
+    // gate/up first
+    if (split) {
+        const int order[2][3] = {{0, 1, 2}, {2, 0, 1}};
+        for (int m = 0; m < 2 && !rc; m++)
+            for (int q = 0; q < PF_NC && !rc; q++) {
+                const int k = order[big_first][q];
+                rc = gemm(m, k, st[k == 2]);
+            }
+    } else {
+        for (int m = 0; m < 2 && !rc; m++)
+            for (int q = PF_NC - 1; q >= 0 && !rc; q--) rc = gemm(m, q, s);
     }
     // recorded even after a failed launch, so that s can always join the side stream
-    if (split && hipEventRecord((hipEvent_t)L->pf_ev[1], ss) != hipSuccess && !rc) rc = K3X_E_HIP;
+    if (split && hipEventRecord((hipEvent_t)L->pf_ev[1], (hipStream_t)L->pf_side) != hipSuccess && !rc)
+        rc = K3X_E_HIP;
     if (rc) PF_RET(rc);
-    if (mx) hipLaunchKernelGGL((pf_gemm_mx<1, DN_RT32, MX_CT_B, false, MX_NW>), dim3(grid_b[1]), dim3(MX_NW * WAVE), 0, s, db);
-    else if (L->special & 4) launch_dn<true, DN_CT32_B, NW_B>(db, grid_b[1], s);
-    else                     launch_dn<false, DN_CT32_B, NW_B>(db, grid_b[1], s);
-    if ((rc = launch_ok())) PF_RET(rc);
-    // the small experts' rows are in y: join the side stream
+    // every routed row is in y: join the side stream
     if (split && hipStreamWaitEvent(s, (hipEvent_t)L->pf_ev[1], 0) != hipSuccess) return K3X_E_HIP;
 
     int sh_row0 = -1;
