@@ -1,6 +1,6 @@
 // k3x_prefill.hip - the prefill path of the MoE block (more than 8 tokens per call):
 //
-//   pf_split    activations to bf16 hi/lo rows (the GEMMs' B source); clears the histogram
+//   pf_rows     fp32 activations to bf16 hi and lo rows (the GEMMs' B source)
 //   pf_router   router logits of every (token, expert) in double, with a bound on their
 //               distance from the reference's chain (k3_router, k3_ops.c:1666-1688)
 //   pf_topk     sigmoid, + bias (:1691-1692), each token's top-k by one wave (:1700-1716),
@@ -9,7 +9,6 @@
 //               the per-expert histogram
 //   pf_scan     per-expert offsets (prefix sum) and the GEMM tile lists
 //   pf_scatter  each (token, slot) to its row in its expert's segment
-//   pf_gather   the routed input's planes, rows in that order
 //   pf_gemm32   grouped GEMMs: gate/up of every expert segment with SwiGLU and the
 //               routing weight (k3_matmul_mxfp4 :3323-3776, k3_situ_glu :148-161), then
 //               down (pf_gemm_mx in the MXFP8 mode)
@@ -31,126 +30,34 @@
 
 #define PF_NT 256
 
-// ------------------------------------------------------------------ split
-// Activation planes, the GEMMs' B source: x [T][H] (bf16 or fp32, rows ldx elements
-// apart) -> xg [2][H/8][T][8] bf16, plane 0 the hi parts, plane 1 the lo parts, each
-// k-group of 8 elements token-major, so that one k-group of consecutive rows is
-// contiguous.  For bf16 rows the lo parts are zero and no GEMM reads plane 1 (they take
-// one column per token, HL = 1): it is not written.  A workgroup transposes a tile of
-// SP_T tokens by SP_G k-groups through LDS, so that both its reads (along the rows) and
-// its writes (along the tokens of a k-group) are contiguous.  Block 0 also clears the
-// expert histogram (when given).
-#define SP_T 32
-#define SP_G 32
-
-static inline unsigned pf_split_grid(int T, int H)
+// ------------------------------------------------------------------ rows
+// The GEMMs' B source is rows of bf16: a bf16 call's activations as they are, and of fp32
+// ones (z in the latent form among them) the hi and the lo rows that this kernel writes,
+// x [T][ldx] fp32 -> hi [T][n], then lo [T][n].  bf16 x: rows copied (strided trunk rows).
+__global__ void __launch_bounds__(PF_NT) pf_rows(const void *x, int x_bf16, int T, int n, int ldx,
+                                                 uint16_t *hl)
 {
-    return (unsigned)(((T + SP_T - 1) / SP_T) * (((H >> 3) + SP_G - 1) / SP_G));
-}
-
-__global__ void __launch_bounds__(PF_NT) pf_split(const void *x, int x_bf16, int T, int H,
-                                                  int ldx, uint16_t *xg, int *counts, int E)
-{
-    __shared__ u32x4 sh[2][SP_G][SP_T + 1];
-    if (blockIdx.x == 0 && counts)
-        for (int e = threadIdx.x; e < E; e += PF_NT) counts[e] = 0;
-    const int G8 = H >> 3, ntg = (G8 + SP_G - 1) / SP_G;
-    const int t0 = (blockIdx.x / ntg) * SP_T, g0 = (blockIdx.x % ntg) * SP_G;
-#pragma unroll
-    for (int j = 0; j < SP_T * SP_G / PF_NT; j++) {
-        const int i = j * PF_NT + threadIdx.x, r = i / SP_G, g = i % SP_G;
-        const int t = t0 + r, gi = g0 + g;
-        u32x4 h = {0u, 0u, 0u, 0u}, l = {0u, 0u, 0u, 0u};
-        const size_t src = (size_t)t * ldx + (size_t)gi * 8;
-        if (t < T && gi < G8 && x_bf16) {
-            h = *(const u32x4 *)((const uint16_t *)x + src);        // bf16: hi = x, lo = 0
-        } else if (t < T && gi < G8) {
-            float v[8];
-            load_x8(x, 0, src, v);
-            uint32_t hi[8], lo[8];
-#pragma unroll
-            for (int k = 0; k < 8; k++) split_bf16(v[k], hi[k], lo[k]);
-#pragma unroll
-            for (int k = 0; k < 4; k++) {
-                h[k] = hi[2 * k] | (hi[2 * k + 1] << 16);
-                l[k] = lo[2 * k] | (lo[2 * k + 1] << 16);
-            }
-        }
-        sh[0][g][r] = h;
-        sh[1][g][r] = l;
+    const int n8 = n >> 3;
+    const size_t f = (size_t)blockIdx.x * PF_NT + threadIdx.x;
+    if (f >= (size_t)T * n8) return;
+    const size_t t = f / n8, c = (f % n8) * 8;
+    if (x_bf16) {
+        *(u32x4 *)(hl + t * n + c) = ld16((const uint16_t *)x + t * ldx + c);
+        return;
     }
-    __syncthreads();
+    float v[8];
+    load_x8(x, 0, t * ldx + c, v);
+    uint32_t hi[8], lo[8];
 #pragma unroll
-    for (int j = 0; j < SP_T * SP_G / PF_NT; j++) {
-        const int i = j * PF_NT + threadIdx.x, g = i / SP_T, r = i % SP_T;
-        const int t = t0 + r, gi = g0 + g;
-        if (t < T && gi < G8) {
-            *(u32x4 *)(xg + ((size_t)gi * T + t) * 8) = sh[0][g][r];
-            if (!x_bf16) *(u32x4 *)(xg + ((size_t)(G8 + gi) * T + t) * 8) = sh[1][g][r];
-        }
+    for (int k = 0; k < 8; k++) split_bf16(v[k], hi[k], lo[k]);
+    u32x4 h, l;
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        h[k] = hi[2 * k] | (hi[2 * k + 1] << 16);
+        l[k] = lo[2 * k] | (lo[2 * k + 1] << 16);
     }
-}
-
-// ------------------------------------------------------------------ gather
-// The routed experts' input planes in permuted order: xg[h][g][p][8] = part h of
-// x[rowmap[p]][8g .. 8g+7], the layout pf_split writes, for TK rows.  A lane owns one
-// permuted row p (consecutive lanes, consecutive p: each store of a k-group is 1 KB
-// contiguous per wave) and walks PG_GS k-groups of its source row, eight at a time: the
-// eight 16-byte pieces of a row's consecutive k-groups (32-byte for fp32 rows) share
-// cache lines, so the walk reads every line once.  The row map is read once per lane
-// and no LDS transpose is needed.
-#define PG_GS 56
-
-static inline unsigned pf_gather_grid(int TK, int H)
-{
-    const int ns = ((H >> 3) + PG_GS - 1) / PG_GS;
-    return (unsigned)((((TK + WAVE - 1) / WAVE) * ns + PF_NT / WAVE - 1) / (PF_NT / WAVE));
-}
-
-__global__ void __launch_bounds__(PF_NT) pf_gather(const void *x, int x_bf16, int TK, int H,
-                                                   int ldx, uint16_t *xg, const int *rowmap)
-{
-    const int G8 = H >> 3, ns = (G8 + PG_GS - 1) / PG_GS;
-    const int w = blockIdx.x * (PF_NT / WAVE) + (int)(threadIdx.x / WAVE);
-    const int pb = w / ns, sl = w % ns;
-    const int p = pb * WAVE + (int)(threadIdx.x % WAVE);
-    if (p >= TK) return;
-    const size_t row = (size_t)rowmap[p] * ldx;
-    const int g0 = sl * PG_GS, g1 = min(G8, g0 + PG_GS);
-    const size_t plane = (size_t)G8 * TK * 8;
-    // G8 is a multiple of 16 (H of 128), so every step of 8 k-groups is whole
-    for (int g = g0; g < g1; g += 8) {
-        if (x_bf16) {
-            u32x4 v[8];
-#pragma unroll
-            for (int j = 0; j < 8; j++) v[j] = ld16((const uint16_t *)x + row + (size_t)(g + j) * 8);
-#pragma unroll
-            for (int j = 0; j < 8; j++) *(u32x4 *)(xg + ((size_t)(g + j) * TK + p) * 8) = v[j];
-        } else {
-            f32x4 v[8][2];
-#pragma unroll
-            for (int j = 0; j < 8; j++) {
-                const float *src = (const float *)x + row + (size_t)(g + j) * 8;
-                v[j][0] = *(const f32x4 *)src;
-                v[j][1] = *(const f32x4 *)(src + 4);
-            }
-#pragma unroll
-            for (int j = 0; j < 8; j++) {
-                uint32_t hi[8], lo[8];
-#pragma unroll
-                for (int k = 0; k < 8; k++) split_bf16(v[j][k >> 2][k & 3], hi[k], lo[k]);
-                u32x4 h, l;
-#pragma unroll
-                for (int k = 0; k < 4; k++) {
-                    h[k] = hi[2 * k] | (hi[2 * k + 1] << 16);
-                    l[k] = lo[2 * k] | (lo[2 * k + 1] << 16);
-                }
-                const size_t o = ((size_t)(g + j) * TK + p) * 8;
-                *(u32x4 *)(xg + o) = h;
-                *(u32x4 *)(xg + plane + o) = l;
-            }
-        }
-    }
+    *(u32x4 *)(hl + t * n + c) = h;
+    *(u32x4 *)(hl + ((size_t)T + t) * n + c) = l;
 }
 
 // ------------------------------------------------------------------ router
@@ -203,6 +110,7 @@ struct PfRouterArgs {
     float       *logit, *gap;
     double      *psum;
     float       *pbnd;
+    int         *counts;             // [E] histogram that the top-k adds to, cleared here
 };
 
 typedef double f64x4 __attribute__((ext_vector_type(4)));
@@ -230,6 +138,8 @@ __global__ void __launch_bounds__(RM_NT, 3) pf_router(PfRouterArgs a)
     constexpr int XL = BF ? 1 : 2;                           // 16-byte loads of 8 activations
     __shared__ double sd[RM_NW][NV][WAVE];
     __shared__ float  sb[RM_NW][NV][WAVE];
+    if (blockIdx.x == 0 && a.counts)
+        for (int e = threadIdx.x; e < a.E; e += RM_NT) a.counts[e] = 0;
     const int nEB = (a.E + RM_E - 1) / RM_E, nTB = (a.T + TT - 1) / TT;
     const int eb = blockIdx.x % nEB, tb = (blockIdx.x / nEB) % nTB, sg = blockIdx.x / (nEB * nTB);
     const int e0 = eb * RM_E, t0 = tb * TT;
@@ -389,7 +299,6 @@ struct PfTopkArgs {
     float        routed_scale;
     int         *idx;   float *wt;       // [T][K]
     int         *uidx;  float *uwt;      // optional caller copies
-    int         *counts;                 // [E] histogram
 };
 
 // The reference's logit of (token t, expert e), one double chain over i = 0 .. H-1
@@ -464,7 +373,7 @@ __global__ void __launch_bounds__(TK_W * WAVE) pf_topk(PfTopkArgs a)
     const int wave = wave_id(), lane = threadIdx.x % WAVE;
     const int T = a.r.T, E = a.r.E, H = a.r.H;
     const int t = blockIdx.x * TK_W + wave;
-    if (a.counts)
+    if (a.r.counts)
         for (int e = threadIdx.x; e < E; e += TK_W * WAVE) hist[e] = 0;
     __syncthreads();
     if (t < T) {                                       // uniform over the wave
@@ -567,13 +476,13 @@ __global__ void __launch_bounds__(TK_W * WAVE) pf_topk(PfTopkArgs a)
             a.idx[o] = e;
             a.wt[o] = s_w[wave][lane];
             if (a.uidx) { a.uidx[o] = e; a.uwt[o] = s_w[wave][lane]; }
-            if (a.counts) atomicAdd(&hist[e], 1);
+            if (a.r.counts) atomicAdd(&hist[e], 1);
         }
     }
-    if (!a.counts) return;                               // uniform
+    if (!a.r.counts) return;                               // uniform
     __syncthreads();
     for (int e = threadIdx.x; e < E; e += TK_W * WAVE)
-        if (hist[e]) atomicAdd(&a.counts[e], hist[e]);
+        if (hist[e]) atomicAdd(&a.r.counts[e], hist[e]);
 }
 
 // ------------------------------------------------------------------ scan
@@ -732,9 +641,13 @@ __global__ void __launch_bounds__(PF_NT) pf_tiles(const int *counts, const int *
 // of the block is in LDS and the slot used by the previous step is free), refills that
 // slot and runs the step's MFMAs.
 //
-// B sources are activation planes [2][K/8][rows][8] bf16 (hi, lo; each k-group
-// row-major over rows), so the 16-byte pieces of one k-group over consecutive rows are
-// contiguous.
+// B sources are bf16 rows [HL][brows][ldb] (hi, then lo).  A load to LDS takes whole runs
+// of a row (256 bytes of a quad of 128 k, 128 of pf_dense's 64), the 16-byte k-groups of
+// column c in the order pos ^ f(c), so that the LDS reads of one k-group over 16
+// consecutive columns fall into distinct banks.  (Planes [2][K/8][rows][8], with a gather
+// of the routed rows into their permuted order, read LDS the same way but cost that pass:
+// 145 us of a 2048-token chunk at the K2 shape, 354 of the latent one, 32 to 57 us of a
+// small call, where it was bound by latency.)
 struct PfGemmArgs {
     const uint8_t  *wm[2];      // group 0's matrices (gate, up) or (down), tiled
     size_t          gstride;    // bytes between groups' records
@@ -744,12 +657,13 @@ struct PfGemmArgs {
     const int      *ntile;      // tiles in this launch's list
     const int      *dbase;      // the list starts at desc + *dbase, or NULL: at desc
     int             n0;
-    const uint16_t *bsrc;       // B planes [2][K/8][brows][8] bf16
-    int             brows;      // rows of each B plane
+    const uint16_t *bsrc;       // B rows [HL][brows][ldb] bf16
+    int             brows;      // rows of each part
+    int             ldb;        // elements between rows
     const int      *perm;       // B row of permuted row p, or NULL: row_base + p
     int             row_base;
     const float    *pw;         // weight of permuted row p (gate/up epilogue), or NULL: 1
-    uint16_t       *act;        // gate/up output planes [2][R/8][arows][8] bf16
+    uint16_t       *act;        // gate/up output rows [2][arows][R] bf16 (hi, lo)
     int             arows;
     float          *y;          // down output rows [*][R] fp32
     int             out_base;   // output row = out_base + p
@@ -768,15 +682,15 @@ struct PfGemmArgs {
 // One dense product Y[p][r] = sum_k W[r][k] B[p][k] with bf16 weights (the shared
 // experts, the latent projections, the trunk matrices): W in the 16-row tile layout
 // (per 128-k quad, 16-byte runs at t*1024 + (row + 16*kq)*16 for k = 32kq + 8t .. +7), B
-// the activation planes.  Both operands go through LDS, fetched by loads straight to LDS,
+// the activation rows.  Both operands go through LDS, fetched by loads straight to LDS,
 // so that every weight byte a workgroup reads serves all of its columns and every B byte
 // all of its rows; the four waves (2 x 2) take RW x CW tiles of 32 x 32 each (NMAT
 // matrices: gate and up of the same rows together) on v_mfma_f32_32x32x16_bf16.
 //
 // K advances 64 at a time through a ring of NS stages.  A stage holds the workgroup's
-// A block as [matrix][k-group g][row][8] and its B block as [g][column][8] (16-byte runs),
-// so that the 32 lanes of an MFMA operand that share a k-group read 512 consecutive
-// bytes.  Each step waits for its stage (the loads issued after it are the NS - 2 stages
+// A block as [matrix][k-group g][row][8] (16-byte runs), so that the 32 lanes of an MFMA
+// operand that share a k-group read 512 consecutive bytes, and its B block as
+// [column][g ^ (column / 2 % 8)][8].  Each step waits for its stage (the loads issued after it are the NS - 2 stages
 // ahead: stages past the end load out of range, which reads nothing and keeps the count
 // exact), meets the other waves, refills the stage freed by the previous step and runs
 // its 16 k-steps' MFMAs.
@@ -822,8 +736,8 @@ __global__ void __launch_bounds__(PF_NT) pf_dense(PfGemmArgs a)
     for (int m = 0; m < NMAT; m++)
         ra[m] = make_rsrc(a.wm[m] + (size_t)t16 * tbytes, ntl * tbytes);
     // load j of a stage: 16-byte run c = j*256 + tid -> (matrix, g, row) of the A block,
-    // or (g, column) of the B block; its offset in the stage's source, less the stage's
-    // own step (A: (st>>1)*4096 + (st&1)*512, B: st*8 k-groups)
+    // or (column, position) of the B block; its offset in the stage's source, less the
+    // stage's own step (A: (st>>1)*4096 + (st&1)*512, B: st*128 bytes)
     uint32_t aoff[NJA], boff[NJB];
 #pragma unroll
     for (int j = 0; j < NJA; j++) {
@@ -832,17 +746,15 @@ __global__ void __launch_bounds__(PF_NT) pf_dense(PfGemmArgs a)
         aoff[j] = (uint32_t)(r >> 4) * tbytes + (uint32_t)(g & 3) * 1024u +
                   (uint32_t)((r & 15) + 16 * (g >> 2)) * 16u;
     }
-    const int G8 = a.K >> 3;
-    const rsrc_t rbs = make_rsrc(a.bsrc, (uint32_t)((size_t)HL * G8 * a.brows * 16));
+    const rsrc_t rbs = make_rsrc(a.bsrc, (uint32_t)((size_t)HL * a.brows * a.ldb * 2));
 #pragma unroll
     for (int j = 0; j < NJB; j++) {
         const int c = j * PF_NT + tid;
-        const int g = c / BN, col = c % BN, tok = col / HL, hl = col % HL;
-        boff[j] = tok < ntok ? ((uint32_t)(hl * G8 + g) * (uint32_t)a.brows +
-                                (uint32_t)(a.row_base + p0 + tok)) * 16u
+        const int col = c >> 3, g = (c & 7) ^ ((col >> 1) & 7), tok = col / HL, hl = col % HL;
+        boff[j] = tok < ntok ? (uint32_t)(hl * a.brows + a.row_base + p0 + tok) * (uint32_t)a.ldb * 2u +
+                                   (uint32_t)g * 16u
                              : K3X_OOB;
     }
-    const uint32_t bstep = (uint32_t)a.brows * 128u;          // 8 k-groups of B
 
     auto ld = [&](int slot, int st) AI {
         const bool on = st < nst;
@@ -861,8 +773,8 @@ __global__ void __launch_bounds__(PF_NT) pf_dense(PfGemmArgs a)
 #pragma unroll
         for (int j = 0; j < NJB; j++) {
             // (a column past the tokens keeps an out-of-range offset: K3X_OOB plus at most
-            // K/64 steps of brows*128 bytes stays below 2^32 and past the planes)
-            const uint32_t o = on ? boff[j] + (uint32_t)st * bstep : K3X_OOB;
+            // K/64 steps of 128 bytes stays below 2^32 and past the rows)
+            const uint32_t o = on ? boff[j] + (uint32_t)st * 128u : K3X_OOB;
             __builtin_amdgcn_raw_ptr_buffer_load_lds(
                 rbs, (lds_void *)(base + SA + (j * PF_NT + wave * WAVE) * 16), 16, o, 0, 0, 0);
         }
@@ -887,7 +799,8 @@ __global__ void __launch_bounds__(PF_NT) pf_dense(PfGemmArgs a)
             bf16x8 bf[CW];
 #pragma unroll
             for (int c = 0; c < CW; c++)
-                bf[c] = as_bf16x8(*(const u32x4 *)(base + SA + (g * BN + (wc * CW + c) * 32 + l32) * 16));
+                bf[c] = as_bf16x8(*(const u32x4 *)(base + SA + ((wc * CW + c) * 32 + l32) * 128 +
+                                                   ((g ^ ((l32 >> 1) & 7)) << 4)));
 #pragma unroll
             for (int m = 0; m < NMAT; m++)
 #pragma unroll
@@ -917,7 +830,6 @@ __global__ void __launch_bounds__(PF_NT) pf_dense(PfGemmArgs a)
     WAIT_VMCNT_LGKM0(0);
 
     // ---- epilogue: lane holds column l32 of each column tile, rows 8aa + 4h + b
-    const int G8o = a.R >> 3;
 #pragma unroll
     for (int c = 0; c < CW; c++) {
         const int col = (wc * CW + c) * 32 + l32;
@@ -944,8 +856,8 @@ __global__ void __launch_bounds__(PF_NT) pf_dense(PfGemmArgs a)
                     uint32_t hi[4], lo[4];
 #pragma unroll
                     for (int b = 0; b < 4; b++) split_bf16(situ(v0[b], v1[b], a.b1, a.b2), hi[b], lo[b]);
-                    const size_t o = ((size_t)(r0 >> 3) * a.arows + (size_t)(a.out_base + p)) * 8 + (r0 & 7);
-                    const size_t plane = (size_t)G8o * a.arows * 8;
+                    const size_t o = (size_t)(a.out_base + p) * a.R + r0;
+                    const size_t plane = (size_t)a.arows * a.R;
                     *(u32x2 *)(a.act + o) = (u32x2){hi[0] | (hi[1] << 16), hi[2] | (hi[3] << 16)};
                     *(u32x2 *)(a.act + plane + o) = (u32x2){lo[0] | (lo[1] << 16), lo[2] | (lo[3] << 16)};
                 } else {
@@ -967,8 +879,8 @@ __global__ void __launch_bounds__(PF_NT) pf_dense(PfGemmArgs a)
 // groups of row R: group kq = h (load 0) and kq = 2 + h (load 1).  Dword d of load g
 // feeds the MFMA of step (g, d) with k = 64g + 32h + 8d .. +7, so one 32x32x16 step
 // multiplies k-slots {64g + 8d .. +7} (lanes 0-31) and {64g + 32 + 8d .. +7} (lanes
-// 32-63).  The B block in LDS is laid out to match: entry ((g*4 + d)*2 + h)*NCOL + col
-// holds those 8 k of column col.  Every product of the quad is formed exactly once;
+// 32-63).  The B block in LDS holds column col's 16 k-groups of the quad at
+// 16 col + (k-group ^ col % 16).  Every product of the quad is formed exactly once;
 // only the order of the fp32 additions differs from the 16x16 form.
 template <bool EXACT, int NMAT, int RT32, int CT32, int HL, bool GU, int NW, int MINW>
 __global__ void __launch_bounds__(NW * WAVE, MINW) pf_gemm32(PfGemmArgs a)
@@ -1041,21 +953,17 @@ __global__ void __launch_bounds__(NW * WAVE, MINW) pf_gemm32(PfGemmArgs a)
     const uint32_t lc = (uint32_t)(Rl >> 4) * tbytes + (uint32_t)((Rl & 15) + 16 * h) * 16u;
     const uint32_t ls = (uint32_t)(Rl >> 4) * tbytes + 4096u + (uint32_t)((Rl & 15) + 16 * h) * 4u;
 
-    // ---- B pieces: entry e = (wave*NJ + j)*64 + lane; e = gdh*NCOL + col,
-    // gdh = (g*4 + d)*2 + h -> k-group 8g + 4h + d of the quad
-    const int G8 = a.K >> 3;
-    const rsrc_t rbs = make_rsrc(a.bsrc, (uint32_t)((size_t)2 * G8 * a.brows * 16));
-    const uint32_t qstep = (uint32_t)a.brows * 256u;
+    // ---- B pieces: entry e = (wave*NJ + j)*64 + lane = 16 col + pos, k-group pos ^ col%16
+    const rsrc_t rbs = make_rsrc(a.bsrc, (uint32_t)((size_t)HL * a.brows * a.ldb * 2));
     uint32_t boff[NJ];
 #pragma unroll
     for (int j = 0; j < NJ; j++) {
         const int e = (wave * NJ + j) * WAVE + lane;
-        const int gdh = e / NCOL, col = e % NCOL;
-        const int gg = gdh >> 3, dd = (gdh >> 1) & 3, hh = gdh & 1;
+        const int col = e >> 4, kg = (e ^ col) & 15;
         const int tok = col / HL, hl = col % HL;
         if (tok < ntok) {
             const int row = a.perm ? a.perm[p0 + tok] : a.row_base + p0 + tok;
-            boff[j] = ((uint32_t)(hl * G8 + 8 * gg + 4 * hh + dd) * (uint32_t)a.brows + (uint32_t)row) * 16u;
+            boff[j] = (uint32_t)(hl * a.brows + row) * (uint32_t)a.ldb * 2u + (uint32_t)kg * 16u;
         } else {
             boff[j] = K3X_OOB;
         }
@@ -1084,7 +992,7 @@ __global__ void __launch_bounds__(NW * WAVE, MINW) pf_gemm32(PfGemmArgs a)
                 }
 #pragma unroll
         for (int j = 0; j < NJ; j++) {
-            const uint32_t o = boff[j] + (uint32_t)q * qstep;
+            const uint32_t o = boff[j] + (uint32_t)q * 256u;
             __builtin_amdgcn_raw_ptr_buffer_load_lds(
                 rbs, (lds_void *)(sB + slot * QB + (wave * NJ + j) * 1024), 16, o, 0, 0, 0);
         }
@@ -1100,6 +1008,8 @@ __global__ void __launch_bounds__(NW * WAVE, MINW) pf_gemm32(PfGemmArgs a)
 #pragma unroll
                 for (int v = 0; v < 16; v++) acc[m][i][c][v] = 0.f;
 
+    // k-group 8 gl + 4 h + d of column Rl (the two xor terms share no bits with it)
+    const int bl = Rl * 256 + (((4 * h) ^ (Rl & 15)) << 4);
     auto compute = [&](int slot, int q) AI {
         const uint8_t *bb = sB + slot * QB;
         const int sh = 8 * (q & 3);
@@ -1118,7 +1028,7 @@ __global__ void __launch_bounds__(NW * WAVE, MINW) pf_gemm32(PfGemmArgs a)
                 bf16x8 bf[CT32];
 #pragma unroll
                 for (int c = 0; c < CT32; c++)
-                    bf[c] = as_bf16x8(*(const u32x4 *)(bb + (((gl * 4 + d) * 2 + h) * NCOL + c * 32 + Rl) * 16));
+                    bf[c] = as_bf16x8(*(const u32x4 *)(bb + c * 8192 + (bl ^ ((8 * gl + d) << 4))));
 #pragma unroll
                 for (int m = 0; m < NMAT; m++)
 #pragma unroll
@@ -1155,7 +1065,6 @@ __global__ void __launch_bounds__(NW * WAVE, MINW) pf_gemm32(PfGemmArgs a)
     WAIT_VMCNT_LGKM0(0);
 
     // ---- epilogue: lane holds column Rl of each column tile, rows 8a + 4h + b
-    const int G8o = a.R >> 3;
 #pragma unroll
     for (int c = 0; c < CT32; c++) {
         const int col = c * 32 + Rl;
@@ -1186,8 +1095,8 @@ __global__ void __launch_bounds__(NW * WAVE, MINW) pf_gemm32(PfGemmArgs a)
                         const float yv = (w == 0.0f) ? 0.0f : w * situ(v0[b], v1[b], a.b1, a.b2);
                         split_bf16(yv, hi[b], lo[b]);
                     }
-                    const size_t o = ((size_t)(r0 >> 3) * a.arows + (size_t)(a.out_base + p)) * 8 + (r0 & 7);
-                    const size_t plane = (size_t)G8o * a.arows * 8;
+                    const size_t o = (size_t)(a.out_base + p) * a.R + r0;
+                    const size_t plane = (size_t)a.arows * a.R;
                     *(u32x2 *)(a.act + o) = (u32x2){hi[0] | (hi[1] << 16), hi[2] | (hi[3] << 16)};
                     *(u32x2 *)(a.act + plane + o) = (u32x2){lo[0] | (lo[1] << 16), lo[2] | (lo[3] << 16)};
                 } else {
@@ -1547,11 +1456,10 @@ __global__ void __launch_bounds__(NW * WAVE) pf_gemm_mx(PfGemmArgs a)
 // ------------------------------------------------------------------ latent norm
 // The latent form's aggregates (agg [T][X], one workgroup per token): RMSNorm with the
 // latent norm weights (k3_rmsnorm, k3_ops.c:132-140 and :1946; double sum of squares, inv
-// rounded to float, w*x*inv), or none when nw is NULL, then the hi and lo parts for the
-// up projection: planes [2][X/8][T][8] (pf_split's layout) for the dense kernel, or with
-// rows set, rows [2][T][X] for the library GEMMs.
+// rounded to float, w*x*inv), or none when nw is NULL, then the hi and lo rows [2][T][X]
+// for the up projection.
 __global__ void __launch_bounds__(PF_NT) pf_latnorm(const float *agg, const float *nw, float eps,
-                                                    int T, int X, uint16_t *hl, int rows)
+                                                    int T, int X, uint16_t *hl)
 {
     __shared__ double red[PF_NT / WAVE];
     __shared__ float s_inv;
@@ -1589,13 +1497,8 @@ __global__ void __launch_bounds__(PF_NT) pf_latnorm(const float *agg, const floa
             h[j] = hi[2 * j] | (hi[2 * j + 1] << 16);
             l[j] = lo[2 * j] | (lo[2 * j + 1] << 16);
         }
-        if (rows) {
-            *(u32x4 *)(hl + (size_t)t * X + (size_t)gi * 8) = h;
-            *(u32x4 *)(hl + ((size_t)T + t) * X + (size_t)gi * 8) = l;
-        } else {
-            *(u32x4 *)(hl + ((size_t)gi * T + t) * 8) = h;
-            *(u32x4 *)(hl + ((size_t)(G8 + gi) * T + t) * 8) = l;
-        }
+        *(u32x4 *)(hl + (size_t)t * X + (size_t)gi * 8) = h;
+        *(u32x4 *)(hl + ((size_t)T + t) * X + (size_t)gi * 8) = l;
     }
 }
 
@@ -1703,6 +1606,13 @@ static inline unsigned round8(size_t n) { return (unsigned)((n + 7) & ~(size_t)7
 #define DENSE_RW    2
 #define DENSE_CW    2
 
+static int launch_rows(const void *x, int x_bf16, int T, int n, int ldx, uint16_t *hl, hipStream_t s)
+{
+    hipLaunchKernelGGL(pf_rows, dim3(cdiv((size_t)T * (n >> 3), PF_NT)), dim3(PF_NT), 0, s, x, x_bf16,
+                       T, n, ldx, hl);
+    return launch_ok();
+}
+
 // A dense product on pf_dense: NMAT matrices of R rows over a.n0 B rows, HL B columns per
 // row (1: bf16 activations, 2: hi and lo parts of fp32 ones)
 template <int NMAT, int RW, int CW, bool GU>
@@ -1730,7 +1640,7 @@ static void launch_router(const PfRouterArgs &a, hipStream_t s)
 }
 
 // Router and top-k of T rows: idx and wt, copies in uidx and uwt, the histogram in counts
-// (cleared before; all three may be NULL).
+// (all three may be NULL).
 static int route_rows(k3x_moe_layer *L, const k3x_prefill_buf *B, const void *x, int x_bf16, int T,
                       int *idx, float *wt, int *uidx, float *uwt, int *counts, hipStream_t s)
 {
@@ -1741,8 +1651,8 @@ static int route_rows(k3x_moe_layer *L, const k3x_prefill_buf *B, const void *x,
     PfRouterArgs &ar = at.r;
     ar.x = x; ar.x_bf16 = x_bf16; ar.W = L->router; ar.T = T; ar.H = H; ar.E = E;
     // workgroups along K: up to three a CU (the LDS holds three), each wave at least one
-    // chunk; the parts' sums and bounds lie in the routed input's planes, which are written
-    // after the top-k
+    // chunk; the parts' sums and bounds lie where the MXFP8 mode's codes are written after
+    // the top-k
     const unsigned tiles = cdiv(E, RM_E) * cdiv(T, 16 * ntt);
     int sg = tiles < 768u / RM_SGMAX ? RM_SGMAX : (tiles < 768u ? (int)(768u / tiles) : 1);
     if (sg > H / RM_KC / RM_NW) sg = H / RM_KC / RM_NW;
@@ -1752,12 +1662,13 @@ static int route_rows(k3x_moe_layer *L, const k3x_prefill_buf *B, const void *x,
     ar.logit = B->logit; ar.gap = B->gap;
     ar.psum = (double *)B->xp;
     ar.pbnd = (float *)(ar.psum + (size_t)ar.sg * T * E);
+    ar.counts = counts;
     if (ntt == 1) launch_router<1>(ar, s);
     else          launch_router<2>(ar, s);
     int rc = launch_ok();
     if (rc) return rc;
     at.bias = L->bias; at.K = K; at.renorm = c->moe_renorm; at.routed_scale = c->routed_scale;
-    at.idx = idx; at.wt = wt; at.uidx = uidx; at.uwt = uwt; at.counts = counts;
+    at.idx = idx; at.wt = wt; at.uidx = uidx; at.uwt = uwt;
     if (E <= 128)      launch_topk<2>(at, s);
     else if (E <= 256) launch_topk<4>(at, s);
     else if (E <= 384) launch_topk<6>(at, s);
@@ -1779,9 +1690,12 @@ static int pf_chunk(k3x_moe_layer *L, const k3x_prefill_buf *B, float *out, cons
     const int HLr = L->lat ? 2 : HLg;                    // of the routed gate/up input
     int rc;
 
-    hipLaunchKernelGGL(pf_split, dim3(pf_split_grid(T, H)), dim3(PF_NT), 0, s,
-                       x, x_bf16, T, H, H, B->xhl, B->counts, E);
-    if ((rc = launch_ok())) return rc;
+    // x's rows as the GEMMs read them
+    const uint16_t *xr = (const uint16_t *)x;
+    if (!x_bf16) {
+        if ((rc = launch_rows(x, 0, T, H, H, B->xhl, s))) return rc;
+        xr = B->xhl;
+    }
 
     // The shared expert (bf16 weights, every token) needs only the split activations: its
     // gate/up and down run on the layer's side stream, beside the dispatch and the routed
@@ -1830,7 +1744,7 @@ static int pf_chunk(k3x_moe_layer *L, const k3x_prefill_buf *B, float *out, cons
         memset(&sg, 0, sizeof sg);
         sg.wm[0] = (const uint8_t *)L->sh_gate; sg.wm[1] = (const uint8_t *)L->sh_up;
         sg.R = SI; sg.K = H; sg.n0 = T;
-        sg.bsrc = B->xhl; sg.brows = T; sg.row_base = 0;
+        sg.bsrc = xr; sg.brows = T; sg.ldb = H; sg.row_base = 0;
         sg.act = B->act_sh; sg.arows = T; sg.out_base = 0;
         sg.b1 = L->b1; sg.b2 = L->b2;
         launch_dense<2, DENSE_GU_RW, DENSE_GU_CW, true>(sg, HLg, side);
@@ -1838,7 +1752,7 @@ static int pf_chunk(k3x_moe_layer *L, const k3x_prefill_buf *B, float *out, cons
         PfGemmArgs sd;
         memset(&sd, 0, sizeof sd);
         sd.wm[0] = (const uint8_t *)L->sh_down; sd.R = H; sd.K = SI; sd.n0 = T;
-        sd.bsrc = B->act_sh; sd.brows = T; sd.row_base = 0;
+        sd.bsrc = B->act_sh; sd.brows = T; sd.ldb = SI; sd.row_base = 0;
         sd.y = B->y; sd.out_base = TK;
         if (!r) {
             launch_dense<1, DENSE_RW, DENSE_CW, false>(sd, 2, side);
@@ -1895,7 +1809,7 @@ static int pf_chunk(k3x_moe_layer *L, const k3x_prefill_buf *B, float *out, cons
             PfGemmArgs zg;
             memset(&zg, 0, sizeof zg);
             zg.wm[0] = (const uint8_t *)L->ldown; zg.R = X; zg.K = H; zg.n0 = T;
-            zg.bsrc = B->xhl; zg.brows = T; zg.row_base = 0;
+            zg.bsrc = xr; zg.brows = T; zg.ldb = H; zg.row_base = 0;
             zg.y = B->zf; zg.out_base = 0;
             launch_dense<1, DENSE_RW, DENSE_CW, false>(zg, HLg, s);
             if ((rc = launch_ok())) PF_RET(rc);
@@ -1909,14 +1823,11 @@ static int pf_chunk(k3x_moe_layer *L, const k3x_prefill_buf *B, float *out, cons
         const void *src = L->lat ? (const void *)B->zf : x;
         hipLaunchKernelGGL(pf_mx8_rows, dim3(pf_mx8_grid(TK, X)), dim3(PF_NT), 0, s,
                            src, L->lat ? 0 : x_bf16, X, X, B->perm_tok, TK, xq8, xs8);
-    } else {
-        // the routed input's planes in permuted order, from x's rows (z's in the latent
-        // form), so that one k-group of an expert's segment is contiguous
-        const void *src = L->lat ? (const void *)B->zf : x;
-        hipLaunchKernelGGL(pf_gather, dim3(pf_gather_grid(TK, X)), dim3(PF_NT), 0, s,
-                           src, L->lat ? 0 : x_bf16, TK, X, X, B->xp, B->perm_tok);
+        if ((rc = launch_ok())) PF_RET(rc);
+    } else if (L->lat) {
+        // z's hi and lo rows (zhl holds the normalised aggregates' only after the GEMMs)
+        if ((rc = launch_rows(B->zf, 0, T, X, X, B->zhl, s))) PF_RET(rc);
     }
-    if ((rc = launch_ok())) PF_RET(rc);
 
     // grids: upper bounds of each class (an expert of class 0 or 1 has one column block;
     // at most TK / (t + 1) experts have more than t tokens); surplus workgroups leave at
@@ -1934,17 +1845,18 @@ static int pf_chunk(k3x_moe_layer *L, const k3x_prefill_buf *B, float *out, cons
         grid[1][0] + grid[1][1] + grid[1][2] > (unsigned)B->ndesc_dn)
         PF_RET(K3X_E_SHAPE);
 
-    // routed gate/up: B rows are the permuted activation rows
+    // routed gate/up: B rows are the tokens' rows, through the permutation
     PfGemmArgs g;
     memset(&g, 0, sizeof g);
     g.wm[0] = L->experts + L->gate_off; g.wm[1] = L->experts + L->up_off;
     g.gstride = L->expert_bytes;
     g.R = I; g.K = X; g.desc = (const int4 *)B->desc_gu;
-    g.bsrc = B->xp; g.brows = TK; g.perm = NULL; g.row_base = 0;
+    g.bsrc = L->lat ? B->zhl : xr; g.brows = T; g.ldb = X; g.perm = B->perm_tok; g.row_base = 0;
     g.pw = B->perm_w; g.act = B->act; g.arows = TK; g.out_base = 0;
     g.b1 = L->b1; g.b2 = L->b2;
     const bool ex_gu = (L->special & 3) != 0;
     if (mx) {
+        g.brows = TK;
         g.b8 = xq8; g.b8s = (const uint32_t *)xs8; g.o8 = aq8; g.o8s = as8;
     }
     // routed down: B rows are the activation rows, in permuted order
@@ -1952,7 +1864,7 @@ static int pf_chunk(k3x_moe_layer *L, const k3x_prefill_buf *B, float *out, cons
     memset(&d, 0, sizeof d);
     d.wm[0] = L->experts + L->down_off; d.gstride = L->expert_bytes;
     d.R = X; d.K = I; d.desc = (const int4 *)B->desc_dn;
-    d.bsrc = B->act; d.brows = TK; d.perm = NULL; d.row_base = 0;
+    d.bsrc = B->act; d.brows = TK; d.ldb = I; d.perm = NULL; d.row_base = 0;
     d.y = B->y; d.out_base = 0;
     if (mx) { d.b8 = aq8; d.b8s = (const uint32_t *)as8; }
     const bool ex_dn = (L->special & 4) != 0;
@@ -2022,19 +1934,17 @@ static int pf_chunk(k3x_moe_layer *L, const k3x_prefill_buf *B, float *out, cons
     const int *pos = B->pos_of;
     int KC = K;
     if (L->lat) {
-        // the routed aggregates in top-k order (:1941-1942), their RMSNorm and hi/lo
-        // planes (:1946), then the up projection (:1950) into y rows 0 .. T-1
+        // the routed aggregates in top-k order (:1941-1942), their RMSNorm's hi and lo rows
+        // (:1946), then the up projection (:1950) into y rows 0 .. T-1
         hipLaunchKernelGGL(pf_combine, dim3(cdiv((size_t)T * (X / 4), PF_NT)), dim3(PF_NT), 0, s,
                            B->y, B->pos_of, T, K, X, -1, (const float *)NULL, B->zf);
         if ((rc = launch_ok())) PF_RET(rc);
         // the up projection: a plain product over the normalised aggregates' hi and lo
-        // parts, on the library where it serves the shapes (rows [T][X] of each part),
-        // else the dense kernel (k-group planes)
+        // rows, on the library where it serves the shapes, else the dense kernel
         const bool up_blas = lib && k3x_blas_ready(L->device, X, H, T, 0) == 0 &&
                              k3x_blas_ready(L->device, X, H, T, 1) == 0;
         hipLaunchKernelGGL(pf_latnorm, dim3(T), dim3(PF_NT), 0, s, B->zf,
-                           c->latent_norm ? L->lnw : (const float *)NULL, c->rms_eps, T, X, B->zhl,
-                           up_blas ? 1 : 0);
+                           c->latent_norm ? L->lnw : (const float *)NULL, c->rms_eps, T, X, B->zhl);
         if ((rc = launch_ok())) PF_RET(rc);
         if (up_blas) {
             if ((rc = k3x_blas_gemm_bf16(L->device, L->lup_rm, X, H, B->y, H, B->zhl, X, T, 0,
@@ -2046,7 +1956,7 @@ static int pf_chunk(k3x_moe_layer *L, const k3x_prefill_buf *B, float *out, cons
             PfGemmArgs ug;
             memset(&ug, 0, sizeof ug);
             ug.wm[0] = (const uint8_t *)L->lup; ug.R = H; ug.K = X; ug.n0 = T;
-            ug.bsrc = B->zhl; ug.brows = T; ug.row_base = 0;
+            ug.bsrc = B->zhl; ug.brows = T; ug.ldb = X; ug.row_base = 0;
             ug.y = B->y; ug.out_base = 0;
             launch_dense<1, DENSE_RW, DENSE_CW, false>(ug, 2, s);
             if ((rc = launch_ok())) PF_RET(rc);
@@ -2112,7 +2022,7 @@ extern "C" int k3x_dev_route(k3x_moe_layer *L, int *idx, float *wt, const void *
 // device holds its own copy at its own address, found once per device by
 // hipGetSymbolAddress; host code uses that address, never the array's name.  Every call
 // on a device shares the device's copy (calls that overlap on one device race); no
-// kernel needs it to start cleared (the histogram is zeroed by pf_split each run).
+// kernel needs it to start cleared (the histogram is zeroed by pf_router each run).
 static __device__ __align__(256) uint8_t scratch[K3X_NOALLOC_BYTES];
 
 #define K3X_MAX_DEVICES 64
@@ -2159,22 +2069,20 @@ extern "C" int k3x_dev_prefill_noalloc(k3x_moe_layer *L, float *out, const void 
 }
 
 // ------------------------------------------------------------------ trunk products
-// Y[t*ldy + o] = W[o] . X[t*ldx] for T activation rows (k3_mmw_batch_ld): X's hi/lo
-// planes into `planes` (T * in * 4 bytes), then the dense bf16 GEMM.
+// Y[t*ldy + o] = W[o] . X[t*ldx] for T activation rows (k3_mmw_batch_ld): X's rows, hi
+// then lo, into `planes` (T * in * 4 bytes), then the dense bf16 GEMM.
 extern "C" int k3x_dev_trunk_gemm(const uint16_t *W, int in, int out, float *y, int ldy,
                                   const void *x, int x_dtype, int ldx, int T, uint16_t *planes,
                                   void *stream)
 {
     hipStream_t s = (hipStream_t)stream;
     const int x_bf16 = (x_dtype == K3X_BF16), HL = x_bf16 ? 1 : 2;
-    hipLaunchKernelGGL(pf_split, dim3(pf_split_grid(T, in)), dim3(PF_NT), 0, s,
-                       x, x_bf16, T, in, ldx, planes, (int *)NULL, 0);
-    int rc = launch_ok();
+    int rc = launch_rows(x, x_bf16, T, in, ldx, planes, s);
     if (rc) return rc;
     PfGemmArgs g;
     memset(&g, 0, sizeof g);
     g.wm[0] = (const uint8_t *)W; g.R = out; g.K = in; g.n0 = T;
-    g.bsrc = planes; g.brows = T; g.row_base = 0;
+    g.bsrc = planes; g.brows = T; g.ldb = in; g.row_base = 0;
     g.y = y; g.out_base = 0; g.ldy = ldy;
     launch_dense<1, DENSE_RW, DENSE_CW, false>(g, HL, s);
     return launch_ok();
