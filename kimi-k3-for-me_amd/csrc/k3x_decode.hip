@@ -700,10 +700,12 @@ __device__ __forceinline__ void bf16_tile_x(const uint16_t *wtile, int K, const 
 }
 
 // One 16-row tile of a tiled bf16 matrix (K columns) times x's compact B set (built by
-// the router launch), staged in LDS: four waves on interleaved quads, as bf16_tile_x, so
-// the same sums; ZR quads of weights in flight a wave (bf16_tile_x keeps two, its ring
-// also holding x's fragments).
+// the router launch): four waves on interleaved quads, as bf16_tile_x, so the same sums;
+// ZR quads of weights in flight a wave (bf16_tile_x keeps two, its ring also holding x's
+// raw rows).  LDSB: the set staged in LDS; else each quad's fragments come from memory with
+// its weights (the set is small and stays in the L2).
 #define ZR 4
+template <bool LDSB>
 __device__ __forceinline__ void bf16_tile_bset(const uint16_t *wtile, int K, const uint16_t *xB,
                                                int NC, float *lds, float (&acc)[4])
 {
@@ -713,23 +715,29 @@ __device__ __forceinline__ void bf16_tile_bset(const uint16_t *wtile, int K, con
     const int cnt = strided_count(wave, NW, nQ);
     const uint32_t bbytes = (uint32_t)nS * 1024u * NC;
     Stage<8> st;
-    st.issue(xB, bbytes, NT1);
+    if (LDSB) st.issue(xB, bbytes, NT1);
     const rsrc_t rw = make_rsrc(wtile, (uint32_t)nQ * 4096u);
-    QB w[ZR];
+    BFrag<LDSB> bf;
+    bf.init(xB, bbytes, NC, lane);
+    QB w[ZR], bg[ZR];
     auto ld = [&](int i, int k) AI {
-        qb_load(w[i], rw, k < cnt ? (uint32_t)(wave + NW * k) * 4096u : K3X_OOB, lane);
+        const int q = wave + NW * k;
+        qb_load(w[i], rw, k < cnt ? (uint32_t)q * 4096u : K3X_OOB, lane);
+        if (!LDSB) {
+#pragma unroll
+            for (int t = 0; t < 4; t++) bg[i].a[t] = bf.get(0u, k < cnt ? q : wave, t);
+        }
     };
     ring_prime<ZR>(ld);
-    st.commit(NT1);
-    __syncthreads();
-    BFrag<true> bf;
-    bf.init(xB, bbytes, NC, lane);
+    if (LDSB) {
+        st.commit(NT1);
+        __syncthreads();
+    }
     f32x4 d = {0.f, 0.f, 0.f, 0.f};
     ring_loop<ZR>(cnt, ld, [&](int i, int k) AI {
-        const int q = wave + NW * k;
         u32x4 b[4];
 #pragma unroll
-        for (int t = 0; t < 4; t++) b[t] = bf.get(0u, q, t);
+        for (int t = 0; t < 4; t++) b[t] = LDSB ? bf.get(0u, wave + NW * k, t) : bg[i].a[t];
         qb_mfma(d, w[i], b);
     });
     acc[0] = d[0]; acc[1] = d[1]; acc[2] = d[2]; acc[3] = d[3];
@@ -738,16 +746,17 @@ __device__ __forceinline__ void bf16_tile_bset(const uint16_t *wtile, int K, con
 
 // The latent down projection z = down . x (k3_mmw_batch, k3_ops.c:1871) for rows
 // 16*rt .. +15, and z's hi/lo B fragments into zB for k2's routed products.  LDSB: x's
-// B set (the router launch's, with the same fragments bf16_tile_x forms from x) staged in
-// LDS, for calls whose set fits (1 or 2 tokens).
+// B set (the router launch's) staged in LDS, for calls whose set fits (1 or 2 tokens).
+// (Past two tokens each workgroup had formed the fragments from x's rows with each quad:
+// 44 us at four fp32 tokens of the K3 shape, now 23 to 27, most of it the selection beside
+// it.)
 template <bool LDSB>
 __device__ void k1_down(const K1Args &a, float *lds, int rt)
 {
     const int wave = wave_id(), lane = threadIdx.x % WAVE;
     const int NC = 2 * a.T;
     float acc[4];
-    if (LDSB) bf16_tile_bset(a.ldown + (size_t)rt * 16 * a.H, a.H, a.xB, NC, lds, acc);
-    else bf16_tile_x(a.ldown + (size_t)rt * 16 * a.H, a.H, a.x, a.x_bf16, a.H, a.T, lds, acc);
+    bf16_tile_bset<LDSB>(a.ldown + (size_t)rt * 16 * a.H, a.H, a.xB, NC, lds, acc);
     // z's set holds whole super-quads; its quads past XL/128 stay zero
     const int nSX = ((a.XL >> 7) + 3) >> 2;
     if (rt == 0)
@@ -1742,14 +1751,8 @@ struct KNArgs {
     uint16_t    *latB;
 };
 
-#define NT4 1024                  // k4_latent_norm: 16 waves, 1024 set entries a workgroup
-
-__device__ __forceinline__ float agg_at(const KNArgs &a, size_t i)
-{
-    float v = a.acc[i];
-    for (int p = 1; p < a.P; p++) v += a.acc[p * a.pstride + i];
-    return v;
-}
+#define NT4 1024                  // k4_latent_norm: 16 waves, a workgroup a token
+#define NL_MAX 14336              // aggregates a workgroup keeps in LDS
 
 // Four consecutive floats at o of each of P parts (pstride floats apart), added in part
 // order.  The loads go out eight parts at a time (a part past P loads the last part again
@@ -1780,62 +1783,60 @@ __device__ __forceinline__ f32x4 agg4(const KNArgs &a, size_t i)
     return parts_sum4(a.acc, a.P, a.pstride, i);
 }
 
+// One workgroup a token: its aggregates (the parts added in order) into LDS, their 1/rms,
+// then the token's two columns of the B set.  Bound by the latency of its three dependent
+// steps.  (A few workgroups dealt the set's entries had each summed every token's parts for
+// the norms, and again for their entries: 37 us at four tokens of the K3 shape, 18 parts;
+// now 11.)  Rows past NL_MAX are added up twice.
 __global__ void __launch_bounds__(NT4) k4_latent_norm(KNArgs a)
 {
-    __shared__ double dl[NT4 / WAVE][K3X_DECODE_MAX_T];
-    __shared__ float s_inv[K3X_DECODE_MAX_T];
-    const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
-    if (a.nw) {
-        // every token's loads of a step in flight together
-        double ss[K3X_DECODE_MAX_T];
-#pragma unroll
-        for (int t = 0; t < K3X_DECODE_MAX_T; t++) ss[t] = 0.0;
+    __shared__ double dl[NT4 / WAVE];
+    __shared__ float s_inv;
+    __shared__ __attribute__((aligned(16))) float agg[NL_MAX];
+    const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE, tok = blockIdx.x;
+    const size_t row = (size_t)tok * a.XL;
+    const bool keep = a.XL <= NL_MAX;
+    double ss = 0.0;
+    if (keep || a.nw)
         for (int i = threadIdx.x * 4; i < a.XL; i += NT4 * 4) {
-#pragma unroll
-            for (int t = 0; t < K3X_DECODE_MAX_T; t++) {
-                if (t >= a.T) break;
-                const f32x4 v = agg4(a, (size_t)t * a.XL + i);
-                ss[t] += (double)v[0] * (double)v[0] + (double)v[1] * (double)v[1] +
-                         (double)v[2] * (double)v[2] + (double)v[3] * (double)v[3];
-            }
+            const f32x4 v = agg4(a, row + i);
+            if (keep) *(f32x4 *)(agg + i) = v;
+            ss += (double)v[0] * (double)v[0] + (double)v[1] * (double)v[1] +
+                  (double)v[2] * (double)v[2] + (double)v[3] * (double)v[3];
         }
-#pragma unroll
-        for (int t = 0; t < K3X_DECODE_MAX_T; t++) {
-            if (t >= a.T) break;
-            double v = ss[t];
-            for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off);
-            if (lane == 0) dl[wave][t] = v;
-        }
-        __syncthreads();
-        if (threadIdx.x < a.T) {
-            double tot = 0.0;
-            for (int w = 0; w < NT4 / WAVE; w++) tot += dl[w][threadIdx.x];
-            s_inv[threadIdx.x] = (float)(1.0 / sqrt(tot / (double)a.XL + (double)a.eps));
-        }
-        __syncthreads();
+    for (int off = 32; off >= 1; off >>= 1) ss += __shfl_xor(ss, off);
+    if (lane == 0) dl[wave] = ss;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        double tot = 0.0;
+        for (int w = 0; w < NT4 / WAVE; w++) tot += dl[w];
+        s_inv = (float)(1.0 / sqrt(tot / (double)a.XL + (double)a.eps));
     }
+    __syncthreads();
     // entries of the compact set (whole super-quads; quads past XL/128 are zeros), as
-    // x_to_bset lays them out
-    const int NC = 2 * a.T, nQ = a.XL >> 7, nq = 4 * (((a.XL >> 7) + 3) >> 2);
-    const int ne = nq * 16 * NC;
-    for (int f = blockIdx.x * NT4 + threadIdx.x; f < ne; f += gridDim.x * NT4) {
-        const int n = f % NC, kq = (f / NC) & 3, t = (f / (NC * 4)) & 3, q = f / (NC * 16);
-        u32x4 v = {0u, 0u, 0u, 0u};
+    // x_to_bset lays them out: hi in column 2 tok, lo beside it
+    const int NC = 2 * a.T, nQ = a.XL >> 7, ne = 4 * ((nQ + 3) >> 2) * 16;
+    for (int f = threadIdx.x; f < ne; f += NT4) {
+        const int kq = f & 3, t = (f >> 2) & 3, q = f >> 4;
+        u32x4 h = {0u, 0u, 0u, 0u}, l = {0u, 0u, 0u, 0u};
         if (q < nQ) {
             const int c0 = q * 128 + kq * 32 + t * 8;
-            const size_t base = (size_t)(n >> 1) * a.XL + c0;
+            const f32x4 v0 = keep ? *(const f32x4 *)(agg + c0) : agg4(a, row + c0);
+            const f32x4 v1 = keep ? *(const f32x4 *)(agg + c0 + 4) : agg4(a, row + c0 + 4);
             float xv[8];
-            const f32x4 v0 = agg4(a, base), v1 = agg4(a, base + 4);
 #pragma unroll
             for (int j = 0; j < 4; j++) { xv[j] = v0[j]; xv[4 + j] = v1[j]; }
             if (a.nw) {
-                const float inv = s_inv[n >> 1];
+                const float inv = s_inv;
 #pragma unroll
                 for (int j = 0; j < 8; j++) xv[j] = a.nw[c0 + j] * xv[j] * inv;
             }
-            v = bfrag_of(xv, n & 1);
+            h = bfrag_of(xv, 0);
+            l = bfrag_of(xv, 1);
         }
-        *(u32x4 *)((uint8_t *)a.latB + (size_t)f * 16) = v;
+        uint8_t *dst = (uint8_t *)a.latB + ((size_t)f * NC + 2 * tok) * 16;
+        *(u32x4 *)dst = h;
+        *(u32x4 *)(dst + 16) = l;
     }
 }
 
@@ -2218,9 +2219,7 @@ extern "C" int k3x_dev_decode(k3x_moe_layer *L, float *out, const void *x, int x
     const bool fuse = k4_lds_bytes(true, false, T, X, L->SI) <= K4_LDS_MAX;
     const bool shl = k4_lds_bytes(fuse, true, T, X, L->SI) <= K4_LDS_MAX;
     if (!fuse) {
-        const int nent = 4 * nSX * 16 * NC;
-        hipLaunchKernelGGL(k4_latent_norm, dim3((nent + NT4 - 1) / NT4), dim3(NT4), 0,
-                           s, an);
+        hipLaunchKernelGGL(k4_latent_norm, dim3(T), dim3(NT4), 0, s, an);
         if ((rc = launch_ok())) return rc;
         if ((rc = record(L, ev++, s))) return rc;
     }
