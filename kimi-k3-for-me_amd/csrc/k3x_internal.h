@@ -181,7 +181,7 @@ struct k3x_moe_layer {
     /* prefill: the shared expert's GEMMs run on a stream of their own, forked from the
      * caller's stream after the activation split and joined before the combine (events
      * 0 and 1); NULL when the layer has no shared expert */
-    void     *pf_side, *pf_ev[2];
+    void     *pf_side, *pf_ev[3];
     int       pf_mode;            /* K3X_PREFILL_EXACT or K3X_PREFILL_MXFP8 */
     size_t    bytes;
     /* decode: bound on the routed workgroups' wait for the published selection (ticks of

@@ -114,6 +114,8 @@ static int layer_alloc(k3x_moe_layer *L)
             hipEventCreateWithFlags((hipEvent_t *)&L->pf_ev[0], hipEventDisableTiming) !=
                 hipSuccess ||
             hipEventCreateWithFlags((hipEvent_t *)&L->pf_ev[1], hipEventDisableTiming) !=
+                hipSuccess ||
+            hipEventCreateWithFlags((hipEvent_t *)&L->pf_ev[2], hipEventDisableTiming) !=
                 hipSuccess)
             return K3X_E_HIP;
     }
@@ -192,7 +194,7 @@ static void layer_free(k3x_moe_layer *L)
     free(L->slot_of); free(L->key_of); free(L->used_at); free(L->pinned);
     for (int i = 0; i < 8; i++)
         if (L->ev[i]) hipEventDestroy((hipEvent_t)L->ev[i]);
-    for (int i = 0; i < 2; i++)
+    for (int i = 0; i < 3; i++)
         if (L->pf_ev[i]) hipEventDestroy((hipEvent_t)L->pf_ev[i]);
     if (L->pf_side) hipStreamDestroy((hipStream_t)L->pf_side);
     free(L);
