@@ -94,6 +94,7 @@ struct KSLds {
     int    need[K3X_DECODE_MAX_T];               // token's selection needs ks_resolve
     int    list[KS_LIST], nlist;                 // ks_resolve's experts of a pass
     alignas(16) double pl[NT / WAVE][KS_CH];     // ks_chain's products
+    TkList tk[NT / WAVE];                        // the waves' selections
 };
 
 // The logit of (token t, expert e) as the reference computes it: one double chain
@@ -189,7 +190,7 @@ __device__ int ks_resolve(const KSArgs &a, KSLds &l, int t, int *s_idx, float *s
         if (wave == 0) {
             float ck;
             wave_topk<NE, 0>(cr, sr, ro, a.E, a.K, a.renorm, a.routed_scale, s_idx, s_w, lane,
-                             out_e, out_w, &ck);
+                             l.tk[0], out_e, out_w, &ck);
             const uint32_t kk = choice_key(ck);
             uint32_t crit = 0u;
 #pragma unroll
@@ -264,7 +265,7 @@ __device__ int ks_route(const KSArgs &a, KSLds &l, bool publish, unsigned seq = 
                                                   __HIP_MEMORY_SCOPE_AGENT);
             float ck;
             wave_topk<NE, 0>(cr, sr, 0u, a.E, a.K, a.renorm, a.routed_scale, l.idx[0], l.w[0],
-                             lane, &ex, &w, &ck);
+                             lane, l.tk[0], &ex, &w, &ck);
             if (lane == 0) {
                 l.need[0] = slack_reaches(hk, ck);
                 if (hk) a.hkey[0] = 0u;      // read: cleared for the next call's router
@@ -322,7 +323,8 @@ __device__ int ks_route(const KSArgs &a, KSLds &l, bool publish, unsigned seq = 
         const uint32_t hk1 = nt == 2 ? __hip_atomic_load(&a.hkey[t1], __ATOMIC_RELAXED,
                                                          __HIP_MEMORY_SCOPE_AGENT) : 0u;
         float ck[2];
-        wave_topk_n<NE, 0, 2>(cr, sr, ro, nt, a.E, a.K, a.renorm, a.routed_scale, si, sw, lane, ck);
+        wave_topk_n<NE, 0, 2>(cr, sr, ro, nt, a.E, a.K, a.renorm, a.routed_scale, si, sw, lane,
+                              l.tk[wave], ck);
         if (lane == 0) {                     // read: cleared for the next call's router
             l.need[wave] = slack_reaches(hk0, ck[0]);
             if (hk0) a.hkey[wave] = 0u;

@@ -91,8 +91,8 @@ __global__ void __launch_bounds__(PF_NT) pf_rows(const void *x, int x_bf16, int 
 // load latency below.  One sequential chain per tile (three waves a SIMD, 48 experts x 64
 // tokens a workgroup) took 229 us at 16 tokens (8 workgroups, the chain's 1792 dependent
 // steps and a load's latency every 64 k), 294 at 301, 302 at 2048 x 384 experts and 774 at
-// 2048 x 896; now 12, 56, 243 and 530, with the top-k 6 -> 14, 8 -> 15, 17 -> 13 and 40 ->
-// 70 us (it adds the parts and works out the sigmoids).
+// 2048 x 896; now 12, 47, 215 and 490, with the top-k (which adds the parts and works out
+// the sigmoids) 6 -> 8, 8 -> 8, 17 -> 6 and 40 -> 16 to 54 us.
 #define RM_E  32
 #define RM_KC 64
 #define RM_NT 256
@@ -116,7 +116,10 @@ struct PfRouterArgs {
 typedef double f64x4 __attribute__((ext_vector_type(4)));
 
 // chunks of segment s of S over H
-__device__ __forceinline__ int rm_seg(int s, int S, int H) { return (int)((long)(H / RM_KC) * s / S); }
+__device__ __forceinline__ int rm_seg(int s, int S, int H)
+{
+    return (int)((unsigned)(H / RM_KC) * (unsigned)s / (unsigned)S);     // s <= 32
+}
 
 // The float logit of a sum v and the distance its chain's float logit can lie from it,
 // given bnd = sum n_s |start_s| + 128 sum B_s.  A sum that is not finite met an infinity
@@ -362,7 +365,7 @@ __device__ double pf_chain(const PfRouterArgs &a, int t, int e, double *buf, int
 // added to the global counts once per workgroup and expert: a device-scope atomic per
 // (token, slot) serialised on the busiest experts' counters (the Zipf chunk's first expert
 // takes every token).
-#define TK_W 8
+#define TK_W 4
 template <int NE>
 __global__ void __launch_bounds__(TK_W * WAVE) pf_topk(PfTopkArgs a)
 {
@@ -370,6 +373,7 @@ __global__ void __launch_bounds__(TK_W * WAVE) pf_topk(PfTopkArgs a)
     __shared__ float    s_w[TK_W][K3X_MAX_TOPK];
     __shared__ int      hist[1024];
     __shared__ __attribute__((aligned(16))) double chain[TK_W][CH_N];
+    __shared__ TkList   list[TK_W];
     const int wave = wave_id(), lane = threadIdx.x % WAVE;
     const int T = a.r.T, E = a.r.E, H = a.r.H;
     const int t = blockIdx.x * TK_W + wave;
@@ -380,16 +384,17 @@ __global__ void __launch_bounds__(TK_W * WAVE) pf_topk(PfTopkArgs a)
         // range-checked loads (an expert past E reads zeros): a load behind a branch would
         // be waited for on its own
         float sc[NE], cv[NE], sl[NE], bi[NE];
-        const uint32_t ro = (uint32_t)(t * E + lane * NE);
+        const uint32_t ro = (uint32_t)(t * E);
         const rsrc_t rb = make_rsrc(a.bias, (uint32_t)E * 4u);
 #pragma unroll
-        for (int c = 0; c < NE; c++) bi[c] = bload_f32<0>(rb, 4u * (uint32_t)(lane * NE + c));
+        for (int c = 0; c < NE; c++) bi[c] = bload_f32<0>(rb, 4u * (uint32_t)(c * WAVE + lane));
         if (a.r.sg == 1) {
             const rsrc_t rl = make_rsrc(a.r.logit, (uint32_t)(T * E) * 4u);
             const rsrc_t rg = make_rsrc(a.r.gap, (uint32_t)(T * E) * 4u);
 #pragma unroll
             for (int c = 0; c < NE; c++) {
-                const uint32_t o = lane * NE + c < E ? 4u * (ro + c) : K3X_OOB;
+                const int e = c * WAVE + lane;
+                const uint32_t o = e < E ? 4u * (ro + e) : K3X_OOB;
                 sc[c] = bload_f32<0>(rl, o);
                 sl[c] = bload_f32<0>(rg, o);
             }
@@ -408,7 +413,8 @@ __global__ void __launch_bounds__(TK_W * WAVE) pf_topk(PfTopkArgs a)
             auto ld = [&](int i, int g) AI {
 #pragma unroll
                 for (int c = 0; c < NE; c++) {
-                    const uint32_t o = ((g < sg) & (lane * NE + c < E)) ? ro + c + (uint32_t)(g * T * E) : K3X_OOB / 8u;
+                    const int e = c * WAVE + lane;
+                    const uint32_t o = ((g < sg) & (e < E)) ? ro + e + (uint32_t)(g * T * E) : K3X_OOB / 8u;
                     v[i][c] = __builtin_amdgcn_raw_buffer_load_b64(rs, 8u * o, 0, 0);
                     w[i][c] = bload_f32<0>(rg, 4u * o);
                 }
@@ -448,12 +454,12 @@ __global__ void __launch_bounds__(TK_W * WAVE) pf_topk(PfTopkArgs a)
         }
         for (;;) {
             float ck;
-            wave_topk_vals<NE>(cv, sc, E, a.K, a.renorm, a.routed_scale, s_idx[wave], s_w[wave],
-                               lane, nullptr, nullptr, &ck);
+            wave_topk_vals<NE, true>(cv, sc, E, a.K, a.renorm, a.routed_scale, s_idx[wave],
+                                     s_w[wave], lane, list[wave], nullptr, nullptr, &ck);
             uint32_t crit = 0u;
 #pragma unroll
             for (int c = 0; c < NE; c++)
-                if (lane * NE + c < E && sl[c] > 0.0f && slack_reaches(slack_key(cv[c], sl[c]), ck))
+                if (c * WAVE + lane < E && sl[c] > 0.0f && slack_reaches(slack_key(cv[c], sl[c]), ck))
                     crit |= 1u << c;
             if (__ballot(crit != 0u) == 0ull) break;
             for (;;) {
@@ -461,7 +467,7 @@ __global__ void __launch_bounds__(TK_W * WAVE) pf_topk(PfTopkArgs a)
                 if (m == 0ull) break;
                 const int l0 = (int)__builtin_ctzll(m);
                 const int cc = __builtin_ctz((uint32_t)__builtin_amdgcn_readlane((int)crit, l0));
-                const float f = (float)pf_chain(a.r, t, l0 * NE + cc, chain[wave], lane);
+                const float f = (float)pf_chain(a.r, t, cc * WAVE + l0, chain[wave], lane);
                 const float s = sigmoid_ref(f);
                 if (lane == l0) crit &= crit - 1u;
 #pragma unroll
@@ -1893,8 +1899,9 @@ static int pf_chunk(k3x_moe_layer *L, const k3x_prefill_buf *B, float *out, cons
             else if (q == 1) ex_dn ? launch_dn<true, 1>(p, gr, st) : launch_dn<false, 1>(p, gr, st);
             else             ex_dn ? launch_dn<true, 2>(p, gr, st) : launch_dn<false, 2>(p, gr, st);
         } else if (HLr == 1) {
-            if (q != 2) ex_gu ? launch_gu<true, 1, 0>(p, gr, st) : launch_gu<false, 1, 0>(p, gr, st);
-            else        ex_gu ? launch_gu<true, 1, 2>(p, gr, st) : launch_gu<false, 1, 2>(p, gr, st);
+            if (q == 0)      ex_gu ? launch_gu<true, 1, 0>(p, gr, st) : launch_gu<false, 1, 0>(p, gr, st);
+            else if (q == 1) ex_gu ? launch_gu<true, 1, 1>(p, gr, st) : launch_gu<false, 1, 1>(p, gr, st);
+            else             ex_gu ? launch_gu<true, 1, 2>(p, gr, st) : launch_gu<false, 1, 2>(p, gr, st);
         } else {
             if (q == 0)      ex_gu ? launch_gu<true, 2, 0>(p, gr, st) : launch_gu<false, 2, 0>(p, gr, st);
             else if (q == 1) ex_gu ? launch_gu<true, 2, 1>(p, gr, st) : launch_gu<false, 2, 1>(p, gr, st);

@@ -82,61 +82,107 @@ __device__ __forceinline__ uint32_t wave_max_u32(uint32_t v)
 
 // One token's top-k by one wave, the reference's repeated maximum (k3_ops.c:1700-1708):
 // K rounds, each taking the largest remaining choice with the lower index first among
-// equal values.  Lane l holds experts l*NE .. l*NE+NE-1 (so a lower lane holds lower
-// indices) as 64-bit words key << 32 | ~index, loaded once (CP: the loads' cache
-// policy); in that order the entries still remaining after a round's winner W are exactly
-// those below W.  A round: each lane's largest word below the previous winner, the wave
-// maximum of their keys, the lowest lane holding it (a ballot: its word has the lowest
-// index among equal keys), and that lane's index and score read as wave-uniform values.
-// Branch-free.  NaN and -inf are never taken; a round with nothing left gives index 0,
-// weight 0.  Weights are the unbiased scores, renormalised through a double sum in slot
-// order and a float reciprocal, then scaled (:1710-1716).  Results in s_idx/s_w, and
-// lane j's (slot j's) in out_e/out_w when given, and the last round's choice (the K-th
-// largest; -inf when fewer than K were selectable) in out_ck.  This form takes the
-// choices and scores in registers (lane l: experts l*NE + c); wave_topk below loads them
-// first.
-template <int NE>
+// equal values; that is the K largest words key << 32 | ~index in order.  Lane l holds
+// experts l*NE + c, or with ST experts c*64 + l (rows of them load coalesced).
+//
+// A bound first: the K-th largest distinct lane maximum, or lower, by K wave maxima (every
+// word of the selection has at least that key).  The words at or above it, K and a few
+// more, go to a list in LDS, and each one's place is the number of listed words above it.
+// Where they are more than the list holds (many equal choices, K near 64), K rounds over
+// all words: each takes the wave's largest word below the previous winner.  (Those rounds
+// for every call walked a lane's NE words each: 64-bit compares, 6700 instructions at 16
+// words and 16 rounds.)  NaN and -inf are never taken; a place that nothing fills gives
+// index 0, weight 0.  Weights are the unbiased scores, renormalised through a double sum
+// in slot order and a float reciprocal, then scaled (:1710-1716).  Results in s_idx/s_w
+// (LDS), and lane j's (slot j's) in out_e/out_w when given, and the K-th largest choice
+// (-inf when fewer than K were selectable) in out_ck.  ts: LDS of this wave.
+struct TkList {
+    uint64_t w[WAVE];
+    float    s[WAVE];
+};
+
+template <int NE, bool ST>
 __device__ void wave_topk_vals(const float (&cv)[NE], const float (&sc)[NE], int E, int K,
                                int renorm, float routed_scale, int *s_idx, float *s_w,
-                               int lane, int *out_e = nullptr, float *out_w = nullptr,
-                               float *out_ck = nullptr)
+                               int lane, TkList &ts, int *out_e = nullptr,
+                               float *out_w = nullptr, float *out_ck = nullptr)
 {
-    uint64_t pk[NE];
+    uint32_t key[NE], lm = 0u, m = 0u;
 #pragma unroll
     for (int c = 0; c < NE; c++) {
-        const int e = lane * NE + c;
         const uint32_t k = choice_key(cv[c]);
-        pk[c] = (e < E && k > K_NEG_INF) ? ((uint64_t)k << 32) | (uint64_t)(~(uint32_t)e) : 0ull;
+        key[c] = ((ST ? c * WAVE + lane : lane * NE + c) < E && k > K_NEG_INF) ? k : 0u;
+        lm = key[c] > lm ? key[c] : lm;
     }
-    uint64_t prev = ~0ull;        // the previous round's winner (none yet: above all)
-    int mine_e = 0;               // lane j keeps round j's expert and score
-    float mine_s = 0.0f;
-    float ck = -__builtin_inff(); // the last round's choice (-inf when a round finds none:
-                                  // the later rounds find none either)
     for (int j = 0; j < K; j++) {
-        uint64_t best = 0ull;
-        float bs = 0.0f;
+        m = wave_max_u32(lm);
+        if (m == 0u) break;                     // uniform
+        lm = lm == m ? 0u : lm;
+    }
+    const uint32_t thr = m ? m : 1u;            // fewer maxima than K: every word
+    int n = 0;
 #pragma unroll
-        for (int c = 0; c < NE; c++) {
-            const uint64_t v = pk[c] < prev ? pk[c] : 0ull;
-            const bool gt = v > best;
-            best = gt ? v : best;
-            bs = gt ? sc[c] : bs;
+    for (int c = 0; c < NE; c++) {
+        const bool on = key[c] >= thr;
+        const uint64_t mask = __ballot(on);
+        const int pos = n + lanes_below(mask);
+        if (on && pos < WAVE) {
+            ts.w[pos] = ((uint64_t)key[c] << 32) |
+                        (uint64_t)(~(uint32_t)(ST ? c * WAVE + lane : lane * NE + c));
+            ts.s[pos] = sc[c];
         }
-        const uint32_t bk = (uint32_t)(best >> 32);
-        const uint32_t m = wave_max_u32(bk);
-        const uint64_t holders = __ballot(m != 0u && bk == m);
-        if (holders == 0ull) {                  // nothing left (uniform)
-            if (lane == j) { mine_e = 0; mine_s = 0.0f; }
-            ck = -__builtin_inff();
-            continue;
+        n += __popcll(mask);
+    }
+    int mine_e = 0;                             // lane j: slot j's expert and score
+    float mine_s = 0.0f;
+    float ck = -__builtin_inff();
+    if (n <= WAVE) {                            // uniform
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        const uint64_t w = lane < n ? ts.w[lane] : 0ull;
+        const float s = lane < n ? ts.s[lane] : 0.0f;
+        int rank = 0;
+        for (int j = 0; j < n; j++) rank += ts.w[j] > w;
+        const bool in = lane < n && rank < K;
+        if (in) {
+            s_idx[rank] = (int)~(uint32_t)w;
+            s_w[rank] = s;
         }
-        const int w = (int)__builtin_ctzll(holders);
-        const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)best, w);
-        const float ws = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(bs), w));
-        prev = ((uint64_t)m << 32) | lo;
-        if (lane == j) { mine_e = (int)~lo; mine_s = ws; }
-        ck = key_choice(m);
+        const uint64_t kth = __ballot(lane < n && rank == K - 1);
+        if (kth != 0ull)
+            ck = key_choice((uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(w >> 32),
+                                                                (int)__builtin_ctzll(kth)));
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        if (lane < n && lane < K) {
+            mine_e = s_idx[lane];
+            mine_s = s_w[lane];
+        }
+    } else {
+        uint64_t prev = ~0ull;    // the previous round's winner (none yet: above all)
+        for (int j = 0; j < K; j++) {
+            uint64_t best = 0ull;
+            float bs = 0.0f;
+#pragma unroll
+            for (int c = 0; c < NE; c++) {
+                const uint64_t pk = ((uint64_t)key[c] << 32) |
+                                    (uint64_t)(~(uint32_t)(ST ? c * WAVE + lane : lane * NE + c));
+                const uint64_t v = key[c] && pk < prev ? pk : 0ull;
+                const bool gt = v > best;
+                best = gt ? v : best;
+                bs = gt ? sc[c] : bs;
+            }
+            const uint32_t bk = (uint32_t)(best >> 32);
+            const uint32_t mk = wave_max_u32(bk);
+            if (mk == 0u) { ck = -__builtin_inff(); break; }    // nothing left (uniform)
+            // the lowest index among the lanes that hold that key
+            const uint32_t lo = bk == mk ? (uint32_t)best : 0u, ml = wave_max_u32(lo);
+            const int w = (int)__builtin_ctzll(__ballot(bk == mk && lo == ml));
+            const float ws = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(bs), w));
+            prev = ((uint64_t)mk << 32) | ml;
+            if (lane == j) { mine_e = (int)~ml; mine_s = ws; }
+            ck = key_choice(mk);
+        }
     }
     if (out_ck) *out_ck = ck;
     float wgt = mine_s;
@@ -155,9 +201,10 @@ __device__ void wave_topk_vals(const float (&cv)[NE], const float (&sc)[NE], int
     if (out_e) { *out_e = mine_e; *out_w = wgt; }
 }
 
+// wave_topk_vals of choices and scores in memory (CP: the loads' cache policy)
 template <int NE, int CP>
 __device__ void wave_topk(rsrc_t cr, rsrc_t sr, uint32_t row_off, int E, int K, int renorm,
-                          float routed_scale, int *s_idx, float *s_w, int lane,
+                          float routed_scale, int *s_idx, float *s_w, int lane, TkList &ts,
                           int *out_e = nullptr, float *out_w = nullptr,
                           float *out_ck = nullptr)
 {
@@ -170,21 +217,18 @@ __device__ void wave_topk(rsrc_t cr, rsrc_t sr, uint32_t row_off, int E, int K, 
         sc[c] = bload_f32<CP>(sr, o);
     }
     SCHED_FENCE();      // both rows' loads in flight together: one memory round trip
-    wave_topk_vals<NE>(cv, sc, E, K, renorm, routed_scale, s_idx, s_w, lane, out_e, out_w,
-                       out_ck);
+    wave_topk_vals<NE, false>(cv, sc, E, K, renorm, routed_scale, s_idx, s_w, lane, ts, out_e,
+                              out_w, out_ck);
 }
 
-// wave_topk for N tokens of one wave together (tokens past ntok load nothing and store
-// nothing): every token's rows are loaded at once (one memory round trip for all), and
-// each round runs for every token before the next, so that one token's wave maximum
-// fills the other's latency.  Per token, the same operations in the same order as
-// wave_topk, so the same results; out_ck[r] is token r's K-th choice.
+// wave_topk for N tokens of one wave (tokens past ntok load nothing and store nothing):
+// every token's rows are loaded at once, one memory round trip for all; out_ck[r] is token
+// r's K-th choice.
 template <int NE, int CP, int N>
 __device__ void wave_topk_n(rsrc_t cr, rsrc_t sr, const uint32_t (&row_off)[N], int ntok, int E,
                             int K, int renorm, float routed_scale, int *const (&s_idx)[N],
-                            float *const (&s_w)[N], int lane, float (&out_ck)[N])
+                            float *const (&s_w)[N], int lane, TkList &ts, float (&out_ck)[N])
 {
-    uint64_t pk[N][NE];
     float sc[N][NE], cv[N][NE];
 #pragma unroll
     for (int r = 0; r < N; r++)
@@ -198,68 +242,9 @@ __device__ void wave_topk_n(rsrc_t cr, rsrc_t sr, const uint32_t (&row_off)[N], 
     SCHED_FENCE();
 #pragma unroll
     for (int r = 0; r < N; r++)
-#pragma unroll
-        for (int c = 0; c < NE; c++) {
-            const int e = lane * NE + c;
-            const uint32_t k = choice_key(cv[r][c]);
-            pk[r][c] = (e < E && k > K_NEG_INF) ? ((uint64_t)k << 32) | (uint64_t)(~(uint32_t)e) : 0ull;
-        }
-    uint64_t prev[N];
-    int mine_e[N];
-    float mine_s[N], ck[N];
-#pragma unroll
-    for (int r = 0; r < N; r++) {
-        prev[r] = ~0ull;
-        mine_e[r] = 0;
-        mine_s[r] = 0.0f;
-        ck[r] = -__builtin_inff();
-    }
-    for (int j = 0; j < K; j++) {
-#pragma unroll
-        for (int r = 0; r < N; r++) {
-            uint64_t best = 0ull;
-            float bs = 0.0f;
-#pragma unroll
-            for (int c = 0; c < NE; c++) {
-                const uint64_t v = pk[r][c] < prev[r] ? pk[r][c] : 0ull;
-                const bool gt = v > best;
-                best = gt ? v : best;
-                bs = gt ? sc[r][c] : bs;
-            }
-            const uint32_t bk = (uint32_t)(best >> 32);
-            const uint32_t m = wave_max_u32(bk);
-            const uint64_t holders = __ballot(m != 0u && bk == m);
-            if (holders == 0ull) {                  // nothing left (uniform)
-                if (lane == j) { mine_e[r] = 0; mine_s[r] = 0.0f; }
-                ck[r] = -__builtin_inff();
-                continue;
-            }
-            const int w = (int)__builtin_ctzll(holders);
-            const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)best, w);
-            const float ws = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(bs), w));
-            prev[r] = ((uint64_t)m << 32) | lo;
-            if (lane == j) { mine_e[r] = (int)~lo; mine_s[r] = ws; }
-            ck[r] = key_choice(m);
-        }
-    }
-#pragma unroll
-    for (int r = 0; r < N; r++) out_ck[r] = ck[r];
-#pragma unroll
-    for (int r = 0; r < N; r++) {
-        float wgt = mine_s[r];
-        if (renorm && K > 1) {
-            double sum = 0.0;
-            for (int j = 0; j < K; j++)
-                sum += (double)__int_as_float(__builtin_amdgcn_readlane(__float_as_int(mine_s[r]), j));
-            const float inv = (float)(1.0 / (sum + 1e-20));
-            wgt *= inv;
-        }
-        wgt *= routed_scale;
-        if (r < ntok && lane < K) {
-            s_idx[r][lane] = mine_e[r];
-            s_w[r][lane] = wgt;
-        }
-    }
+        if (r < ntok)
+            wave_topk_vals<NE, false>(cv[r], sc[r], E, K, renorm, routed_scale, s_idx[r], s_w[r],
+                                      lane, ts, nullptr, nullptr, &out_ck[r]);
 }
 
 #endif
