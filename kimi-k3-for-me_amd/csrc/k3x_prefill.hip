@@ -1624,7 +1624,9 @@ static void launch_dense(const PfGemmArgs &a, int HL, hipStream_t s)
 // wide tiles' workgroups, launched on another stream, find no free CU among class 0's until
 // those end.  (The routed products of 40 fp32 tokens at the K2 shape: 780 us a call with
 // three classes, 680 with one; 130 latent tokens 2482 and 2437; 301 tokens, 6.3 rows an
-// expert, within their noise; from 8 to 16 rows no difference either way.)
+// expert, within their noise; from 8 to 16 rows no difference either way.  In the MXFP8
+// mode, whose class 2 runs on the same stream, 40 tokens 710 and 660, 120 tokens 1188 and
+// 1156.)
 #define PF_ONE_ROWS 8
 // and from which class 2's products are the longer part (at 42.7, the K2 shape's 2048
 // tokens, 3.08 ms with them on the caller's stream and 3.36 on the side stream; at 14.6 no
@@ -1801,7 +1803,7 @@ static int pf_chunk(k3x_moe_layer *L, const k3x_prefill_buf *B, float *out, cons
     sa.counts = B->counts; sa.E = E; sa.offsets = B->offsets; sa.cursor = B->cursor;
     sa.tb[0] = B->tb_gu; sa.tb[1] = B->tb_dn;
     // calls of few tokens an expert: one class for all (see PF_ONE_ROWS)
-    const bool one = !mx && TK < PF_ONE_ROWS * E;
+    const bool one = TK < PF_ONE_ROWS * E;
     const PfShape mgu[PF_NC] = {{MX_NW, MX_GU_RT32_S, MX_CT_S, 0}, {MX_NW, MX_GU_RT32_S, MX_CT_S, 0},
                                 {MX_NW, MX_GU_RT32, MX_CT_B, 0}};
     const PfShape mdn[PF_NC] = {{MX_NW, MX_DN_RT32_S, MX_CT_S, 0}, {MX_NW, MX_DN_RT32_S, MX_CT_S, 0},
