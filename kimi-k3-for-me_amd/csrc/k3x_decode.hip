@@ -1844,8 +1844,8 @@ __global__ void __launch_bounds__(NT4) k4_latent_norm(KNArgs a)
 
 // The up projection (k3_ops.c:1950) of the normalised aggregates and the shared expert's
 // down product (moe_shared, :1858) for 16 output rows: eight waves on interleaved bf16
-// quads of `up` and then of the shared down matrix, into two accumulator sets; out =
-// up + shared (:1859), plus the residual.
+// quads of `up` and then of the shared down matrix, into one accumulator set (:1859); out =
+// the sum, plus the residual.
 //   FUSE: the workgroup works out the aggregates itself, while its first weights are in
 //         flight: the parts of k3 added in order into LDS (fp32), each token's 1/rms, and
 //         the normalised set's B fragments into LDS at 0 (else they come from
@@ -1863,6 +1863,10 @@ struct K4Args {
     int             T, H, XL, SI;
 };
 
+// quads in flight a wave, of either matrix.  (Two of each matrix in rings of their own, the
+// first ring's two alone while `up` streams: 217.5 us a call of two latent tokens, 360 of six
+// fp32 ones; now 212 and 355, other calls within their noise; four in flight 210 and 360.)
+#define K4_R 3
 #define K4_LDS_MAX 65536u          // with the static reduction area, two workgroups per CU
 
 __host__ __device__ inline uint32_t k4_lds_bytes(bool fuse, bool shl, int T, int XL, int SI)
@@ -1920,7 +1924,7 @@ __device__ __forceinline__ void k4_fuse_norm(const KNArgs &a, float *agg, double
 template <bool FUSE, bool SHL>
 __global__ void __launch_bounds__(NT3) k4_up(K4Args a)
 {
-    __shared__ __attribute__((aligned(16))) float lds[(NT3 / WAVE - 1) * 8 * WAVE];
+    __shared__ __attribute__((aligned(16))) float lds[(NT3 / WAVE - 1) * 4 * WAVE];
     __shared__ double dl[NT3 / WAVE][K3X_DECODE_MAX_T];
     __shared__ float s_inv[K3X_DECODE_MAX_T];
     constexpr int NW = NT3 / WAVE;
@@ -1938,48 +1942,55 @@ __global__ void __launch_bounds__(NT3) k4_up(K4Args a)
     const rsrc_t rb1 = make_rsrc(a.latB, lbytes), rb2 = make_rsrc(a.shB, sbytes);
     const int n = lane & 15, kq = lane >> 4;
     const uint32_t boff = (uint32_t)((kq * NC + (n < NC ? n : 0)) * 16);
-    QBB r1[2], r2[2];
-    auto ldq = [&](QBB &it, rsrc_t rw, rsrc_t rb, int k, int cnt, bool gb) AI {
-        const bool on = k < cnt;
-        const int q = wave + NW * k;
-        qb_load(it.a, rw, on ? (uint32_t)q * 4096u : K3X_OOB, lane);
-        if (gb) {
+    // the wave's quads of `up`, then of the shared down matrix, through one ring (K4_R in
+    // flight whichever matrix they belong to) into one accumulator set
+    QBB r[K4_R];
+    const int c12 = c1 + c2;
+    auto ld = [&](int i, int k) AI {
+        const bool up = k < c1, on = k < c12;
+        const int q = wave + NW * (up ? k : k - c1);
+        const uint32_t wo = on ? (uint32_t)q * 4096u : K3X_OOB;
+        qb_load(r[i].a, up ? rw1 : rw2, wo, lane);
+        // fragments from memory where the set is not in LDS (a bound of the other set's
+        // resource: nothing is loaded)
+        if (!FUSE || !SHL) {
+            const bool gb = on && (up ? !FUSE : !SHL);
 #pragma unroll
             for (int t = 0; t < 4; t++)
-                it.b[t] = bload16(rb, on ? boff + (uint32_t)(q * 256 * NC + t * 64 * NC) : K3X_OOB);
+                r[i].b[t] = bload16(up ? rb1 : rb2, gb ? boff + (uint32_t)(q * 256 * NC + t * 64 * NC) : K3X_OOB);
         }
     };
-    auto ld1 = [&](int i, int k) AI { ldq(r1[i], rw1, rb1, k, c1, !FUSE); };
-    auto ld2 = [&](int i, int k) AI { ldq(r2[i], rw2, rb2, k, c2, !SHL); };
-    ring_prime<2>(ld1);
-    ring_prime<2>(ld2);
+    ring_prime<K4_R>(ld);
     if (SHL) st2.commit(NT3, sh_off);
     if (FUSE)
         k4_fuse_norm(a.kn, (float *)(dyn_lds + sh_off + (SHL ? sbytes : 0u)), dl, s_inv);
     if (FUSE || SHL) __syncthreads();
     BFrag<true> bf;
     bf.init(nullptr, 0u, NC, lane);
-    f32x4 d1 = {0.f, 0.f, 0.f, 0.f}, d2 = {0.f, 0.f, 0.f, 0.f};
-    auto use = [&](f32x4 &d, const QBB &it, bool inlds, uint32_t sbase, int q) AI {
-        if (inlds) {
-            u32x4 b[4];
+    f32x4 d = {0.f, 0.f, 0.f, 0.f};
+    ring_loop<K4_R>(c12, ld, [&](int i, int k) AI {
+        const bool up = k < c1;
+        u32x4 b[4];
 #pragma unroll
-            for (int t = 0; t < 4; t++) b[t] = bf.get(sbase, q, t);
-            qb_mfma(d, it.a, b);
-        } else {
-            qb_mfma(d, it.a, it.b);
+        for (int t = 0; t < 4; t++) {
+            if (FUSE && SHL) {
+                b[t] = bf.get(up ? 0u : sh_off, wave + NW * (up ? k : k - c1), t);
+            } else if (FUSE || SHL) {
+                b[t] = r[i].b[t];
+                if (up ? FUSE : SHL) b[t] = bf.get(up ? 0u : sh_off, wave + NW * (up ? k : k - c1), t);
+            } else {
+                b[t] = r[i].b[t];
+            }
         }
-    };
-    ring_loop<2>(c1, ld1, [&](int i, int k) AI { use(d1, r1[i], FUSE, 0u, wave + NW * k); });
-    ring_loop<2>(c2, ld2, [&](int i, int k) AI { use(d2, r2[i], SHL, sh_off, wave + NW * k); });
-    float acc[8] = {d1[0], d1[1], d1[2], d1[3], d2[0], d2[1], d2[2], d2[3]};
-    wave_sum_lds<8, NW>(acc, lds, wave, lane);
+        qb_mfma(d, r[i].a, b);
+    });
+    float acc[4] = {d[0], d[1], d[2], d[3]};
+    wave_sum_lds<4, NW>(acc, lds, wave, lane);
     if (wave != 0) return;
-    per_token<8>(acc, NC, lane, [&](int r0, int tok, const float (&v)[8]) AI {
+    per_token<4>(acc, NC, lane, [&](int r0, int tok, const float (&v)[4]) AI {
         for (int i = 0; i < 4; i++) {
             const size_t o = (size_t)tok * a.H + rt * 16 + r0 + i;
-            const float y = v[i] + v[4 + i];
-            a.out[o] = a.resid ? a.resid[o] + y : y;
+            a.out[o] = a.resid ? a.resid[o] + v[i] : v[i];
         }
     });
 }

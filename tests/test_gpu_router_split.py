@@ -78,3 +78,30 @@ def test_split_router_bitwise(torch, k3x, H, E, K, T, bf16):
             assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), (t, got, want)
     assert np.abs(wt.cpu().numpy() - rw).max() <= 2.0 ** -23
     layer.close()
+
+
+@pytest.mark.parametrize("E,K", [(200, 8), (100, 64), (64, 64), (896, 16)])
+@pytest.mark.parametrize("T", [1, 3, 20])
+def test_equal_choices(torch, k3x, E, K, T):
+    """More equal choices than the selection's list holds, K up to every expert: rows of
+    zeros (every score 0.5) over biases of a few values, the lower index first; a row of
+    N(0, 1) beside them."""
+    say(f"case: equal choices E={E} K={K} T={T}")
+    L = synth.Layer(H=256, E=E, K=K, I=128, n_shared=0, seed=92)
+    L.bias[:] = np.where(np.arange(E) % 3 == 1, 0.25, 0.0).astype(np.float32)
+    L.bias[E - 1] = -np.inf
+    x = L.x(T, bf16=False, stream_sub=92)
+    x[: max(1, T - 1)] = 0.0
+    layer = k3x.MoELayer.from_bank(layer_cfg(k3x, L), L.gate, L.bias, [L.expert(0)] * E)
+    xt = torch.from_numpy(x).cuda()
+    out = torch.empty_like(xt)
+    idx = torch.full((T, K), -7, dtype=torch.int32, device="cuda")
+    wt = torch.full((T, K), -7.0, dtype=torch.float32, device="cuda")
+    layer.forward(out.data_ptr(), xt.data_ptr(), T, k3x.K3X_F32, 0, idx.data_ptr(), wt.data_ptr(),
+                  torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    layer.check()
+    ri, rw = oracle_routes(L, x)
+    assert np.array_equal(idx.cpu().numpy(), ri)
+    assert np.abs(wt.cpu().numpy() - rw).max() <= 2.0 ** -22
+    layer.close()
