@@ -1622,12 +1622,12 @@ static void launch_dense(const PfGemmArgs &a, int HL, hipStream_t s)
 // shape, a larger one in several column blocks (their weights then come from the L2 again),
 // on one stream: a second and third launch each end in a tail of a few workgroups, and the
 // wide tiles' workgroups, launched on another stream, find no free CU among class 0's until
-// those end.  (The routed products of 40 fp32 tokens at the K2 shape: 780 us a call with
-// three classes, 680 with one; 130 latent tokens 2482 and 2437; 301 tokens, 6.3 rows an
-// expert, within their noise; from 8 to 16 rows no difference either way.  In the MXFP8
-// mode, whose class 2 runs on the same stream, 40 tokens 710 and 660, 120 tokens 1188 and
-// 1156.)
-#define PF_ONE_ROWS 8
+// those end.  (The routed products of 40 fp32 tokens at the K2 shape, 0.8 rows an expert:
+// 780 us a call with three classes, 680 with one; 130 latent tokens, 2.3 rows, 2482 and
+// 2437; from 3.3 to 4.6 rows no difference; 250 tokens, 5.2 rows, 1540 and 1608; 350 fp32
+// tokens, 7.3 rows, 1765 and 1838.  In the MXFP8 mode, whose class 2 runs on the same
+// stream, 40 tokens 710 and 660, 120 tokens 1188 and 1156, 300 tokens 1553 and 1569.)
+#define PF_ONE_ROWS 4
 // and from which class 2's products are the longer part (at 42.7, the K2 shape's 2048
 // tokens, 3.08 ms with them on the caller's stream and 3.36 on the side stream; at 14.6 no
 // difference)
