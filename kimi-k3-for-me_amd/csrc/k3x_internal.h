@@ -102,7 +102,7 @@ typedef struct k3x_prefill_buf {
     void     *retired[K3X_PF_RETIRED];
     int       nretired;
     size_t    retired_bytes;
-    uint16_t *xhl;          /* [T][H/8][2][8] bf16 hi/lo activation rows            */
+    uint16_t *xhl;          /* [2][T][H] bf16 hi rows, then lo rows, of fp32 input      */
     float    *logit, *gap;  /* [T][E] router logits, and how far the reference's can lie
                                from each (0: equal)                                   */
     int      *idx;          /* [T][K]                                                */
@@ -114,16 +114,17 @@ typedef struct k3x_prefill_buf {
                                  class its number of tiles and its first            */
     void     *desc_gu, *desc_dn;   /* per GEMM tile {expert, row block, row, rows}      */
     int       ndesc_gu, ndesc_dn;  /* entries of each table                            */
-    uint16_t *xp;           /* [2][H/8][T*K][8] gate/up activations, permuted rows    */
+    uint16_t *xp;           /* the router's partial sums (double [parts][T][E]); after it
+                               the MXFP8 codes and scales of the permuted rows         */
     int      *perm_tok;     /* [T*K] token of each permuted row                      */
     float    *perm_w;       /* [T*K] routing weight of each permuted row             */
     int      *pos_of;       /* [T*K] permuted row of each (token, slot)              */
-    uint16_t *act;          /* [T*K][I/8][2][8] routed activations, hi/lo            */
-    uint16_t *act_sh;       /* [T][SI/8][2][8] shared activations                    */
+    uint16_t *act;          /* [2][T*K][I] routed activations, hi rows then lo rows  */
+    uint16_t *act_sh;       /* [2][T][SI] shared activations                         */
     float    *y;            /* [T*K + T][H] expert and shared output rows            */
     /* latent form (X = latent width) */
     float    *zf;           /* [T][X] z = down . x, then the routed aggregates        */
-    uint16_t *zhl;          /* [2][X/8][T][8] hi/lo planes of the normalised
+    uint16_t *zhl;          /* [2][T][X] hi and lo rows of z, then of the normalised
                                aggregates                                             */
     int       no_lib;       /* 1: no library GEMMs (the no-allocation entry point: a
                                library call may load code objects into device memory) */

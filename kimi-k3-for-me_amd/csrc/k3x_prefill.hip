@@ -1816,6 +1816,27 @@ static int pf_chunk(k3x_moe_layer *L, const k3x_prefill_buf *B, float *out, cons
             sa.nrb[m][q] = cdiv(m ? X : I, p.nw * p.rt * 32);
             if (q < 2) sa.lim[m][q] = one ? TK : sa.tpb[m][q];
         }
+    // grids: upper bounds of each class (an expert of class 0 or 1 has one column block;
+    // at most TK / (t + 1) experts have more than t tokens); surplus workgroups leave at
+    // once
+    unsigned grid[2][PF_NC];
+    for (int m = 0; m < 2; m++) {
+        const size_t ne = E < TK ? E : TK;
+        size_t n[PF_NC] = {ne, (size_t)TK / (sa.lim[m][0] + 1), (size_t)TK / (sa.lim[m][1] + 1)};
+        for (int q = 1; q < PF_NC; q++) n[q] = n[q] < ne ? n[q] : ne;
+        if (sa.lim[m][1] == sa.lim[m][0]) n[1] = 0;
+        size_t tiles = 0;
+        for (int q = 0; q < PF_NC; q++) {
+            if (n[q] && (q == 2 || sa.lim[m][q] > sa.tpb[m][q])) n[q] += cdiv(TK, sa.tpb[m][q]);
+            tiles += sa.nrb[m][q] * n[q];
+            grid[m][q] = round8(sa.nrb[m][q] * n[q]);
+        }
+        // (before any descriptor is written.  The table counts a column block per 16 rows and
+        // one more per expert, each of ceil(rows / 64) row blocks, where a class has at least
+        // 16 rows a column block and 128 a row block: the bound stays below it)
+        if (tiles > (size_t)(m ? B->ndesc_dn : B->ndesc_gu)) PF_RET(K3X_E_SHAPE);
+    }
+
     hipLaunchKernelGGL(pf_scan, dim3(1), dim3(1024), 0, s, sa);
     if ((rc = launch_ok())) PF_RET(rc);
     hipLaunchKernelGGL(pf_scatter, dim3(cdiv(TK, PF_NT)), dim3(PF_NT), 0, s, B->idx, B->wt, TK, K,
@@ -1842,23 +1863,6 @@ static int pf_chunk(k3x_moe_layer *L, const k3x_prefill_buf *B, float *out, cons
         // z's hi and lo rows (zhl holds the normalised aggregates' only after the GEMMs)
         if ((rc = launch_rows(B->zf, 0, T, X, X, B->zhl, s))) PF_RET(rc);
     }
-
-    // grids: upper bounds of each class (an expert of class 0 or 1 has one column block;
-    // at most TK / (t + 1) experts have more than t tokens); surplus workgroups leave at
-    // once
-    unsigned grid[2][PF_NC];
-    for (int m = 0; m < 2; m++) {
-        const size_t ne = E < TK ? E : TK;
-        size_t n[PF_NC] = {ne, (size_t)TK / (sa.lim[m][0] + 1), (size_t)TK / (sa.lim[m][1] + 1)};
-        for (int q = 1; q < PF_NC; q++) n[q] = n[q] < ne ? n[q] : ne;
-        if (sa.lim[m][1] == sa.lim[m][0]) n[1] = 0;
-        for (int q = 0; q < PF_NC; q++)
-            if (n[q] && (q == 2 || sa.lim[m][q] > sa.tpb[m][q])) n[q] += cdiv(TK, sa.tpb[m][q]);
-        for (int q = 0; q < PF_NC; q++) grid[m][q] = round8(sa.nrb[m][q] * n[q]);
-    }
-    if (grid[0][0] + grid[0][1] + grid[0][2] > (unsigned)B->ndesc_gu ||
-        grid[1][0] + grid[1][1] + grid[1][2] > (unsigned)B->ndesc_dn)
-        PF_RET(K3X_E_SHAPE);
 
     // routed gate/up: B rows are the tokens' rows, through the permutation
     PfGemmArgs g;

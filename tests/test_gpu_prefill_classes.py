@@ -49,3 +49,19 @@ def test_one_expert_takes_every_token(torch, k3x):
     assert (oi[:, 0] == 5).all() and np.array_equal(idx, oi)
     assert synth.rel_l2(out, o) < 2e-5
     layer.close()
+
+
+@pytest.mark.parametrize("E,K,T,H,I,bf16", [(1, 1, 17, 256, 256, False), (3, 2, 9, 128, 256, True),
+                                            (2, 2, 16, 128, 128, False), (5, 1, 93, 384, 128, False),
+                                            (4, 1, 33, 128, 128, True)])
+def test_few_experts(torch, k3x, E, K, T, H, I, bf16):
+    """Calls whose launch grids, rounded up to the XCDs, exceed the tile table: the table is
+    held against the tiles themselves."""
+    L = synth.Layer(H=H, E=E, K=K, I=I, seed=19)
+    layer = bank_layer(k3x, L)
+    x = L.x(T, bf16=bf16, stream_sub=19)
+    o, oi, _, _ = L.oracle_moe(x)
+    out, idx, _ = dev_forward(torch, k3x, layer, x, bf16=bf16)
+    assert np.array_equal(idx, oi)
+    assert synth.rel_l2(out, o) < 2e-5
+    layer.close()
