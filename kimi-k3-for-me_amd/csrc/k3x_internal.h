@@ -121,7 +121,8 @@ typedef struct k3x_prefill_buf {
     int      *pos_of;       /* [T*K] permuted row of each (token, slot)              */
     uint16_t *act;          /* [2][T*K][I] routed activations, hi rows then lo rows  */
     uint16_t *act_sh;       /* [2][T][SI] shared activations                         */
-    float    *y;            /* [T*K + T][H] expert and shared output rows            */
+    float    *y;            /* T*K expert output rows of X floats, and from T*K * max(X, H) on
+                               the T shared expert's rows of H                         */
     /* latent form (X = latent width) */
     float    *zf;           /* [T][X] z = down . x, then the routed aggregates        */
     uint16_t *zhl;          /* [2][T][X] hi and lo rows of z, then of the normalised

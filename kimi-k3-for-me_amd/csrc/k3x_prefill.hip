@@ -1510,10 +1510,10 @@ __global__ void __launch_bounds__(PF_NT) pf_latnorm(const float *agg, const floa
 }
 
 // ------------------------------------------------------------------ combine
-// out[t] = ((y[pos(t,0)] + y[pos(t,1)]) + ... ) + y_shared[t], then + resid (pos_of
-// NULL: K = 1 and row t).
+// out[t] = ((y[pos(t,0)] + y[pos(t,1)]) + ... ) + ysh[t], then + resid (pos_of NULL: K = 1
+// and row t; ysh NULL: none).
 __global__ void __launch_bounds__(PF_NT) pf_combine(const float *y, const int *pos_of, int T, int K,
-                                                    int H, int sh_row0, const float *resid,
+                                                    int H, const float *ysh, const float *resid,
                                                     float *out)
 {
     const size_t i = (size_t)blockIdx.x * PF_NT + threadIdx.x;
@@ -1525,8 +1525,8 @@ __global__ void __launch_bounds__(PF_NT) pf_combine(const float *y, const int *p
         const size_t row = pos_of ? (size_t)pos_of[(size_t)t * K + j] : (size_t)t;
         s += *(const f32x4 *)(y + row * H + h);
     }
-    if (sh_row0 >= 0) s += *(const f32x4 *)(y + (size_t)(sh_row0 + t) * H + h);
     const size_t o = (size_t)t * H + h;
+    if (ysh) s += *(const f32x4 *)(ysh + o);
     if (resid) s += *(const f32x4 *)(resid + o);
     *(f32x4 *)(out + o) = s;
 }
@@ -1709,8 +1709,10 @@ static int pf_chunk(k3x_moe_layer *L, const k3x_prefill_buf *B, float *out, cons
     // shared expert is forked after it (3.26 to 3.30 ms at 2048 tokens against 3.37 to
     // 3.46), and after the small classes' products where those are on the side stream, so
     // that these, bound by HBM, run beside the wide tiles, bound by the matrix cores (3.05
-    // to 3.06 ms against 3.10 to 3.15).  Its T rows follow the TK routed rows in y, which
-    // nothing on s writes.
+    // to 3.06 ms against 3.10 to 3.15).
+    // Its T output rows (H floats each) lie in y past the TK routed rows (X floats each) and
+    // past rows of H floats, which the latent form's up projection writes: X may be the wider.
+    float *const ysh = B->y + (size_t)TK * (X > H ? X : H);
     bool forked = false;
     // The library path (bf16 rows, 2*SI <= H, a kernel for each shape): the gate/up product
     // into fp32 rows [T][2*SI] held in the shared rows of y (nothing else writes them before
@@ -1744,7 +1746,6 @@ static int pf_chunk(k3x_moe_layer *L, const k3x_prefill_buf *B, float *out, cons
 #define PF_RET(e) do { const int e_ = (e); (void)join(); return e_; } while (0)
     auto shared = [&]() -> int {
         if (sh_blas) {
-            float *ysh = B->y + (size_t)TK * H;
             uint16_t *ahi = B->act_sh, *alo = B->act_sh + (size_t)T * SI;
             int r = k3x_blas_gemm_bf16(L->device, L->sh_gu_rm, H, 2 * SI, ysh, 2 * SI,
                                        (const uint16_t *)x, H, T, 0, side);
@@ -1769,7 +1770,7 @@ static int pf_chunk(k3x_moe_layer *L, const k3x_prefill_buf *B, float *out, cons
         memset(&sd, 0, sizeof sd);
         sd.wm[0] = (const uint8_t *)L->sh_down; sd.R = H; sd.K = SI; sd.n0 = T;
         sd.bsrc = B->act_sh; sd.brows = T; sd.ldb = SI; sd.row_base = 0;
-        sd.y = B->y; sd.out_base = TK;
+        sd.y = ysh; sd.out_base = 0;
         launch_dense<1, DENSE_RW, DENSE_CW, false>(sd, 2, side);
         return launch_ok();
     };
@@ -1943,14 +1944,14 @@ static int pf_chunk(k3x_moe_layer *L, const k3x_prefill_buf *B, float *out, cons
     if (rc) PF_RET(rc);
     if (split && L->lat && (rc = join())) return rc;     // every routed row is in y
 
-    int sh_row0 = -1;
     const int *pos = B->pos_of;
     int KC = K;
     if (L->lat) {
         // the routed aggregates in top-k order (:1941-1942), their RMSNorm's hi and lo rows
         // (:1946), then the up projection (:1950) into y rows 0 .. T-1
         hipLaunchKernelGGL(pf_combine, dim3(cdiv((size_t)T * (X / 4), PF_NT)), dim3(PF_NT), 0, s,
-                           B->y, B->pos_of, T, K, X, -1, (const float *)NULL, B->zf);
+                           B->y, B->pos_of, T, K, X, (const float *)NULL, (const float *)NULL,
+                           B->zf);
         if ((rc = launch_ok())) PF_RET(rc);
         // the up projection: a plain product over the normalised aggregates' hi and lo
         // rows, on the library where it serves the shapes, else the dense kernel
@@ -1979,10 +1980,9 @@ static int pf_chunk(k3x_moe_layer *L, const k3x_prefill_buf *B, float *out, cons
     }
     // the shared rows (and the side stream's routed ones) are in y
     if ((rc = join())) return rc;
-    if (SI > 0) sh_row0 = TK;
 
     hipLaunchKernelGGL(pf_combine, dim3(cdiv((size_t)T * (H / 4), PF_NT)), dim3(PF_NT), 0, s,
-                       B->y, pos, T, KC, H, sh_row0, resid, out);
+                       B->y, pos, T, KC, H, SI > 0 ? ysh : (const float *)NULL, resid, out);
     return launch_ok();
 }
 #undef PF_RET
