@@ -89,10 +89,12 @@ __global__ void __launch_bounds__(PF_NT) pf_rows(const void *x, int x_bf16, int 
 // summed in LDS; where the tiles are few, gridDim gives each to SG workgroups as well,
 // whose parts pf_topk adds.  Bound by the FP64 matrix cores past a few hundred tokens, by
 // load latency below.  One sequential chain per tile (three waves a SIMD, 48 experts x 64
-// tokens a workgroup) took 229 us at 16 tokens (8 workgroups, the chain's 1792 dependent
-// steps and a load's latency every 64 k), 294 at 301, 302 at 2048 x 384 experts and 774 at
-// 2048 x 896; now 12, 47, 215 and 490, with the top-k (which adds the parts and works out
-// the sigmoids) 6 -> 8, 8 -> 8, 17 -> 6 and 40 -> 16 to 54 us.
+// tokens a workgroup) made a routing call, router and top-k, 226 us at 16 tokens x 384 experts
+// (8 workgroups, the chain's 1792 dependent steps and a load's latency every 64 k), 227 at 301,
+// 229 at 1500, 231 at 2048 and 615 at 2048 x 896; now 20, 55, 208, 250 and 509.  It was the
+// faster only where its tiles fill a round of the CUs (1700 to 2048 x 384, and twice that, by
+// 2 to 10%).  (Tried at 2048 x 384 and within 2% of this: 64 tokens a wave, P_c by a float
+// MFMA instead of shuffles, each workgroup starting its segments at another chunk.)
 #define RM_E  32
 #define RM_KC 64
 #define RM_NT 256
@@ -1654,9 +1656,19 @@ static int route_rows(k3x_moe_layer *L, const k3x_prefill_buf *B, const void *x,
     ar.x = x; ar.x_bf16 = x_bf16; ar.W = L->router; ar.T = T; ar.H = H; ar.E = E;
     // workgroups along K: up to three a CU (the LDS holds three), each wave at least one
     // chunk; the parts' sums and bounds lie where the MXFP8 mode's codes are written after
-    // the top-k
+    // the top-k.  Past one tile a CU, the number of up to four whose last round of workgroups
+    // over the CUs is the fullest, a part's store and load (12 bytes an output) weighed
+    // against its products: with one workgroup a tile there 1500 tokens x 384 experts took
+    // the three rounds of 2048 (a routing call 250 us, now 208; 600 x 896 255, now 212)
     const unsigned tiles = cdiv(E, RM_E) * cdiv(T, 16 * ntt);
-    int sg = tiles < 768u / RM_SGMAX ? RM_SGMAX : (tiles < 768u ? (int)(768u / tiles) : 1);
+    int sg = tiles < 768u / RM_SGMAX ? RM_SGMAX : (int)(768u / tiles);
+    if (tiles > 256u) {
+        double best = 0.0;
+        for (int q = 1; q <= 4; q++) {
+            const double cost = (double)cdiv((size_t)tiles * q, 256) / q + (q > 1 ? 8e-5 * tiles * q : 0.0);
+            if (q == 1 || cost < best) { best = cost; sg = q; }
+        }
+    }
     if (sg > H / RM_KC / RM_NW) sg = H / RM_KC / RM_NW;
     const size_t room = (size_t)T * K * (L->XL > H ? L->XL : H) * 4 / ((size_t)T * E * 12);
     if ((size_t)sg > room) sg = (int)room;
