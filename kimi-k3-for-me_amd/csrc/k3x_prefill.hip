@@ -1556,6 +1556,10 @@ struct PfShape { int nw, rt, ct, minw; };
 static constexpr PfShape GU1[PF_NC] = {{4, 2, 1, 2}, {4, 2, 1, 2}, {8, 1, 3, 2}};   // bf16 rows
 static constexpr PfShape GU2[PF_NC] = {{4, 1, 1, 3}, {8, 1, 2, 2}, {8, 1, 3, 2}};   // hi and lo columns
 static constexpr PfShape DN[PF_NC] = {{4, 2, 1, 3}, {4, 2, 2, 2}, {8, 2, 3, 2}};
+// Classes 0 and 1 and class 2 run on two streams, gate/up then down with no event between
+// them: an expert has to be of class 2 in both products or in neither.
+static_assert(GU1[1].ct * 32 == DN[1].ct * 16 && GU2[1].ct * 16 == DN[1].ct * 16,
+              "the most tokens of class 1 differ between gate/up and down");
 
 template <bool EXACT, int HL, int C>
 static void launch_gu(const PfGemmArgs &a, unsigned grid, hipStream_t s)
