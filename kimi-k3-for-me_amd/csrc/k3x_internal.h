@@ -54,6 +54,7 @@ extern "C" {
 #define K3X_STAGE_MAX    65536   /* bytes of activation fragments a workgroup stages in LDS */
 #define K3X_MAX_TOPK     64      /* K3_MAX_TOPK, k3.h:857-864 */
 #define K3X_ROUTE_WAIT_DEFAULT 100000000ull  /* 1 s at 100 MHz: decode's bound on the wait */
+#define K3X_PF_PARTS     8       /* most parts of K a prefill router's tile is cut into */
 #define K3X_PF_CHUNK     4096    /* prefill: most tokens per pipeline run */
 #define K3X_NOALLOC_BYTES (64u << 20)  /* the no-allocation prefill's static device array */
 #define K3X_CACHE_IO     8       /* expert-cache misses read from the store concurrently */
@@ -114,8 +115,9 @@ typedef struct k3x_prefill_buf {
                                  class its number of tiles and its first            */
     void     *desc_gu, *desc_dn;   /* per GEMM tile {expert, row block, row, rows}      */
     int       ndesc_gu, ndesc_dn;  /* entries of each table                            */
-    uint16_t *xp;           /* the router's partial sums (double [parts][T][E]); after it
-                               the MXFP8 codes and scales of the permuted rows         */
+    uint8_t  *xp;           /* the router's partial sums (double [parts][T][E], then float);
+                               after it the MXFP8 codes and scales of the permuted rows
+                               (k3x_pf_xp_bytes)                                      */
     int      *perm_tok;     /* [T*K] token of each permuted row                      */
     float    *perm_w;       /* [T*K] routing weight of each permuted row             */
     int      *pos_of;       /* [T*K] permuted row of each (token, slot)              */
@@ -256,6 +258,11 @@ int k3x_pf_reserve(struct k3x_moe_layer *L, int T, void *stream);
 /* The prefill buffers of runs of T tokens carved from p (256-byte aligned regions) into
  * B; returns the bytes they take (with p or B NULL, only that) (k3x_moe.c) */
 size_t k3x_pf_layout(const struct k3x_moe_layer *L, int T, char *p, k3x_prefill_buf *B);
+/* bytes of xp for runs of T tokens: the larger of the MXFP8 codes and scales of the T*K
+ * routed rows and the router's parts (12 bytes a logit, K3X_PF_PARTS of them where they fit
+ * xp_rows); and xp_rows, T*K fp32 rows of the widest activation (k3x_moe.c) */
+size_t k3x_pf_xp_bytes(const struct k3x_moe_layer *L, int T);
+size_t k3x_pf_xp_rows(const struct k3x_moe_layer *L, int T);
 /* the prefill pipeline over one run of T <= the chunk tokens with its working buffers
  * in the static device array, never allocating (k3x_prefill.hip) */
 int k3x_dev_prefill_noalloc(struct k3x_moe_layer *L, float *out, const void *x, int x_dtype,

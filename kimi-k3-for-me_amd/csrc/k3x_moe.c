@@ -955,6 +955,21 @@ int k3x_pf_reserve(k3x_moe_layer *L, int T, void *stream)
     return 0;
 }
 
+size_t k3x_pf_xp_rows(const k3x_moe_layer *L, int T)
+{
+    const size_t W = (size_t)(L->XL > L->cfg.hidden ? L->XL : L->cfg.hidden);
+    return (size_t)T * (size_t)L->cfg.topk * W * 4;
+}
+
+size_t k3x_pf_xp_bytes(const k3x_moe_layer *L, int T)
+{
+    const size_t TK = (size_t)T * (size_t)L->cfg.topk, X = (size_t)L->XL;
+    const size_t parts = K3X_PF_PARTS * 12 * (size_t)T * (size_t)L->cfg.n_experts;
+    const size_t rows = k3x_pf_xp_rows(L, T), r = parts < rows ? parts : rows;
+    const size_t mx = ((TK * X + 255) & ~(size_t)255) + TK * (X / 32);
+    return r > mx ? r : mx;
+}
+
 size_t k3x_pf_layout(const k3x_moe_layer *L, int T, char *p, k3x_prefill_buf *B)
 {
     const k3x_cfg *c = &L->cfg;
@@ -976,7 +991,7 @@ size_t k3x_pf_layout(const k3x_moe_layer *L, int T, char *p, k3x_prefill_buf *B)
         t * K * I * 4,             /* act     */
         (SI ? t * SI * 4 : 256),   /* act_sh  */
         (t * K + t) * H * 4,       /* y       */
-        t * K * H * 4,             /* xp      */
+        k3x_pf_xp_bytes(L, T),     /* xp      */
         L->lat ? t * X * 4 : 256,  /* zf      */
         L->lat ? t * X * 4 : 256,  /* zhl     */
         (size_t)ndg * 16,          /* desc_gu */
@@ -1000,7 +1015,7 @@ size_t k3x_pf_layout(const k3x_moe_layer *L, int T, char *p, k3x_prefill_buf *B)
     B->pos_of = (int *)(p + off[12]);
     B->act = (uint16_t *)(p + off[13]); B->act_sh = (uint16_t *)(p + off[14]);
     B->y = (float *)(p + off[15]);
-    B->xp = (uint16_t *)(p + off[16]);
+    B->xp = (uint8_t *)(p + off[16]);
     B->zf = (float *)(p + off[17]);     B->zhl = (uint16_t *)(p + off[18]);
     B->desc_gu = p + off[19]; B->ndesc_gu = ndg;
     B->desc_dn = p + off[20]; B->ndesc_dn = ndd;

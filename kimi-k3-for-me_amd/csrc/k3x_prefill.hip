@@ -99,7 +99,7 @@ __global__ void __launch_bounds__(PF_NT) pf_rows(const void *x, int x_bf16, int 
 #define RM_KC 64
 #define RM_NT 256
 #define RM_NW (RM_NT / WAVE)
-#define RM_SGMAX 8
+#define RM_SGMAX K3X_PF_PARTS
 
 struct PfRouterArgs {
     const void  *x;
@@ -1674,7 +1674,7 @@ static int route_rows(k3x_moe_layer *L, const k3x_prefill_buf *B, const void *x,
         }
     }
     if (sg > H / RM_KC / RM_NW) sg = H / RM_KC / RM_NW;
-    const size_t room = (size_t)T * K * (L->XL > H ? L->XL : H) * 4 / ((size_t)T * E * 12);
+    const size_t room = k3x_pf_xp_bytes(L, T) / ((size_t)T * E * 12);
     if ((size_t)sg > room) sg = (int)room;
     ar.sg = sg < 1 ? 1 : sg;
     ar.logit = B->logit; ar.gap = B->gap;
@@ -1869,7 +1869,7 @@ static int pf_chunk(k3x_moe_layer *L, const k3x_prefill_buf *B, float *out, cons
     }
     // MXFP8 mode: the routed input quantised in permuted order, codes then scales in xp;
     // the gate/up output's codes then scales in act
-    uint8_t *xq8 = (uint8_t *)B->xp, *xs8 = xq8 + (((size_t)TK * X + 255) & ~(size_t)255);
+    uint8_t *xq8 = B->xp, *xs8 = xq8 + (((size_t)TK * X + 255) & ~(size_t)255);
     uint8_t *aq8 = (uint8_t *)B->act, *as8 = aq8 + (((size_t)TK * I + 255) & ~(size_t)255);
     if (mx) {
         const void *src = L->lat ? (const void *)B->zf : x;
@@ -2078,7 +2078,9 @@ extern "C" int k3x_dev_prefill_noalloc(k3x_moe_layer *L, float *out, const void 
                                        void *stream)
 {
     const int chunk = k3x_pf_chunk_tokens(L);
-    const size_t need = k3x_pf_layout(L, T, NULL, NULL);
+    // the limit on T as it is published: fp32 rows of every (token, slot) counted for xp
+    const size_t need = k3x_pf_layout(L, T, NULL, NULL) -
+                        ((k3x_pf_xp_bytes(L, T) + 255) & ~(size_t)255) + k3x_pf_xp_rows(L, T);
     if (T > chunk || need > K3X_NOALLOC_BYTES) {
         fprintf(stderr, "k3x: a prefill of %d tokens needs %zu bytes of working memory; the "
                         "static array holds %u (and one run at most %d tokens)\n",
