@@ -661,11 +661,10 @@ struct PfGemmArgs {
     const uint8_t  *wm[2];      // group 0's matrices (gate, up) or (down), tiled
     size_t          gstride;    // bytes between groups' records
     int             R, K;       // rows and inner dimension of each matrix
-    const int4     *desc;       // per tile {group, row block, first row, rows}, or NULL:
-                                // one group of n0 rows
+    const int4     *desc;       // grouped: per tile {group, row block, first row, rows}
     const int      *ntile;      // tiles in this launch's list
-    const int      *dbase;      // the list starts at desc + *dbase, or NULL: at desc
-    int             n0;
+    const int      *dbase;      // the list starts at desc + *dbase
+    int             n0;         // pf_dense: rows
     const uint16_t *bsrc;       // B rows [HL][brows][ldb] bf16
     int             brows;      // rows of each part
     int             ldb;        // elements between rows
@@ -896,8 +895,6 @@ __global__ void __launch_bounds__(NW * WAVE, MINW) pf_gemm32(PfGemmArgs a)
 {
     constexpr int NTH = NW * WAVE;
     constexpr int NCOL = CT32 * 32;
-    constexpr int TPB = NCOL / HL;
-    constexpr int RPB = NW * RT32 * 32;
     constexpr int QB = NCOL * 128 * 2;
     constexpr int NJ = QB / (NTH * 16);
     constexpr int RING = 4;
@@ -911,8 +908,7 @@ __global__ void __launch_bounds__(NW * WAVE, MINW) pf_gemm32(PfGemmArgs a)
     __shared__ __attribute__((aligned(16))) uint8_t sB[RING * QB];
 
     const int wave = wave_id(), lane = threadIdx.x % WAVE;
-    const int nrb = (a.R + RPB - 1) / RPB;
-    int g = 0, rb, ntok, p0;
+    int g, rb, ntok, p0;
     {
         // Workgroups are dealt to the 8 XCDs round-robin; tiles are dealt to them in
         // contiguous runs instead (XCD x takes tiles x*per .. x*per + per-1 in order), so
@@ -921,22 +917,13 @@ __global__ void __launch_bounds__(NW * WAVE, MINW) pf_gemm32(PfGemmArgs a)
         // the descriptor words are read into scalar registers (readfirstlane): the
         // weight resources built from them must be wave-uniform, or every buffer load
         // becomes a loop over distinct descriptors
-        const int ntiles = a.desc ? __builtin_amdgcn_readfirstlane(*a.ntile)
-                                  : nrb * ((a.n0 + TPB - 1) / TPB);
+        const int ntiles = __builtin_amdgcn_readfirstlane(*a.ntile);
         const int per = (ntiles + 7) >> 3;
         const int k = blockIdx.x >> 3, tile = (blockIdx.x & 7) * per + k;
         if (k >= per || tile >= ntiles) return;
-        if (a.desc) {
-            const int4 d = a.desc[(a.dbase ? __builtin_amdgcn_readfirstlane(*a.dbase) : 0) + tile];
-            g = __builtin_amdgcn_readfirstlane(d.x); rb = __builtin_amdgcn_readfirstlane(d.y);
-            p0 = __builtin_amdgcn_readfirstlane(d.z); ntok = __builtin_amdgcn_readfirstlane(d.w);
-        } else {
-            const int nc = (a.n0 + TPB - 1) / TPB;
-            rb = tile / nc;
-            const int cb = tile % nc;
-            p0 = cb * TPB;
-            ntok = min(TPB, a.n0 - p0);
-        }
+        const int4 d = a.desc[__builtin_amdgcn_readfirstlane(*a.dbase) + tile];
+        g = __builtin_amdgcn_readfirstlane(d.x); rb = __builtin_amdgcn_readfirstlane(d.y);
+        p0 = __builtin_amdgcn_readfirstlane(d.z); ntok = __builtin_amdgcn_readfirstlane(d.w);
     }
     const int nQ = a.K >> 7;
 
@@ -1241,7 +1228,6 @@ __global__ void __launch_bounds__(NW * WAVE) pf_gemm_mx(PfGemmArgs a)
 {
     constexpr int NTH = NW * WAVE;
     constexpr int NCOL = CT * 32;
-    constexpr int RPB = NW * RT32 * 32;
     constexpr int QB = 8 * NCOL * 16;
     constexpr int NJ = QB / (NTH * 16);
     constexpr int RING = 4;
@@ -1253,24 +1239,15 @@ __global__ void __launch_bounds__(NW * WAVE) pf_gemm_mx(PfGemmArgs a)
     __shared__ __attribute__((aligned(16))) uint8_t sB[RING * QB];
 
     const int wave = wave_id(), lane = threadIdx.x % WAVE;
-    const int nrb = (a.R + RPB - 1) / RPB;
-    int g = 0, rb, ntok, p0;
+    int g, rb, ntok, p0;
     {
-        const int ntiles = a.desc ? __builtin_amdgcn_readfirstlane(*a.ntile)
-                                  : nrb * ((a.n0 + NCOL - 1) / NCOL);
+        const int ntiles = __builtin_amdgcn_readfirstlane(*a.ntile);
         const int per = (ntiles + 7) >> 3;
         const int k = blockIdx.x >> 3, tile = (blockIdx.x & 7) * per + k;
         if (k >= per || tile >= ntiles) return;
-        if (a.desc) {
-            const int4 d = a.desc[(a.dbase ? __builtin_amdgcn_readfirstlane(*a.dbase) : 0) + tile];
-            g = __builtin_amdgcn_readfirstlane(d.x); rb = __builtin_amdgcn_readfirstlane(d.y);
-            p0 = __builtin_amdgcn_readfirstlane(d.z); ntok = __builtin_amdgcn_readfirstlane(d.w);
-        } else {
-            const int nc = (a.n0 + NCOL - 1) / NCOL;
-            rb = tile / nc;
-            p0 = (tile % nc) * NCOL;
-            ntok = min(NCOL, a.n0 - p0);
-        }
+        const int4 d = a.desc[__builtin_amdgcn_readfirstlane(*a.dbase) + tile];
+        g = __builtin_amdgcn_readfirstlane(d.x); rb = __builtin_amdgcn_readfirstlane(d.y);
+        p0 = __builtin_amdgcn_readfirstlane(d.z); ntok = __builtin_amdgcn_readfirstlane(d.w);
     }
     const int nQ = a.K >> 7;
 
