@@ -182,9 +182,9 @@ struct k3x_moe_layer {
     unsigned long long *tr;
     int       tr_cap, tr_n[3];
     k3x_prefill_buf pf;
-    /* prefill: the shared expert's GEMMs run on a stream of their own, forked from the
-     * caller's stream after the activation split and joined before the combine (events
-     * 0 and 1); NULL when the layer has no shared expert */
+    /* prefill: the side stream (z, the shared expert and one part of the routed products),
+     * forked from the caller's up to three times a run (event 0) and joined before the
+     * combine (event 1; event 2: z); NULL when the layer has no shared expert */
     void     *pf_side, *pf_ev[3];
     int       pf_mode;            /* K3X_PREFILL_EXACT or K3X_PREFILL_MXFP8 */
     size_t    bytes;

@@ -1605,15 +1605,18 @@ static void launch_dense(const PfGemmArgs &a, int HL, hipStream_t s)
 // shape, a larger one in several column blocks (their weights then come from the L2 again),
 // on one stream: a second and third launch each end in a tail of a few workgroups, and the
 // wide tiles' workgroups, launched on another stream, find no free CU among class 0's until
-// those end.  (The routed products of 40 fp32 tokens at the K2 shape, 0.8 rows an expert:
-// 780 us a call with three classes, 680 with one; 130 latent tokens, 2.3 rows, 2482 and
-// 2437; from 3.3 to 4.6 rows no difference; 250 tokens, 5.2 rows, 1540 and 1608; 350 fp32
-// tokens, 7.3 rows, 1765 and 1838.  In the MXFP8 mode, whose class 2 runs on the same
-// stream, 40 tokens 710 and 660, 120 tokens 1188 and 1156, 300 tokens 1553 and 1569.)
+// those end.  (us a call with three classes and with one, K2 shape: 40 fp32 tokens, 0.8 rows
+// an expert, 759 and 665; 100 of bf16, 2.1 rows, 1142 and 1147; 180, 3.8 rows, 1439 and 1475,
+// of fp32 1456 and 1457; 250, 5.2 rows, 1542 and 1587; 350 of fp32, 7.3 rows, 1779 and 1852.
+// 40 latent tokens, 0.7 rows, 1368 and 1300; 130, 2.3 rows, 2400 and 2358; 440, 7.9 rows, 3426
+// and 3493.  MXFP8 mode, whose class 2 runs on the same stream: 40 tokens 736 and 688, 120
+// 1242 and 1226, 180 1446 and 1455, 300 1587 and 1634.)
 #define PF_ONE_ROWS 4
-// and from which class 2's products are the longer part (at 42.7, the K2 shape's 2048
-// tokens, 3.08 ms with them on the caller's stream and 3.36 on the side stream; at 14.6 no
-// difference)
+// and from which class 2's products are the longer part (us a call with them on the caller's
+// stream and on the side stream, K2 shape, bf16 rows: 14.6 rows 2082 and 2030, 17.7 2231 and
+// 2297, 20.8 2338 and 2407, 25 2530 and 2612, 29 2636 and 2672, 35 2940 and 3027, 42.7 3229
+// and 3301; fp32 rows within 1%.  Latent: 19.6 rows 4994 and 4984, 28.6 6339 and 6432, 36.6
+// 7426 and 7572.)
 #define PF_BIG_ROWS 20
 
 template <int NTT>
@@ -1696,13 +1699,13 @@ static int pf_chunk(k3x_moe_layer *L, const k3x_prefill_buf *B, float *out, cons
     // expert (bf16 weights, every token), which need only x's rows, and the part of the
     // routed products that is not on s.  pf_dense's workgroups, two a CU, let the router and
     // the top-k in beside them: z and then a pf_dense shared expert are forked before those
-    // (a 16-token MoE half 0.89 against 0.93 ms, 2048 latent tokens 7.67 against 7.70; z
-    // there 7.19 against 7.22, 130 latent tokens 2.47 against 2.50).  The library's kernels
-    // hold every CU while they run, so that the top-k would wait for a free one: a library
-    // shared expert is forked after it (3.26 to 3.30 ms at 2048 tokens against 3.37 to
-    // 3.46), and after the small classes' products where those are on the side stream, so
-    // that these, bound by HBM, run beside the wide tiles, bound by the matrix cores (3.05
-    // to 3.06 ms against 3.10 to 3.15).
+    // (z here against on s before the routed products: 16 latent tokens 677 and 680 us, of fp32
+    // 726 and 744, 130 2354 and 2372, 600 and 2048 within 0.6%).  The library's kernels hold
+    // every CU while they run, so that the top-k would wait for a free one: a library shared
+    // expert is forked after it (before it, 3 to 5% more at 2048 tokens when the routed input was
+    // still gathered), and after the small
+    // classes' products where those are on the side stream (there against before them: 1000
+    // tokens 2333 and 2344 us, 1400 2630 and 2667, 2048 3239 and 3234).
     // Its T output rows (H floats each) lie in y past the TK routed rows (X floats each) and
     // past rows of H floats, which the latent form's up projection writes: X may be the wider.
     float *const ysh = B->y + (size_t)TK * (X > H ? X : H);
@@ -1911,9 +1914,13 @@ static int pf_chunk(k3x_moe_layer *L, const k3x_prefill_buf *B, float *out, cons
     };
     // In the exact mode the products of classes 0 and 1 and those of class 2 run on two
     // streams, s and the side stream (forked here, after the routed input is written; joined
-    // before the combine): 3.56 to 3.58 against 3.61 ms per 2048-token chunk.  The longer of
-    // the two goes on s.  The MXFP8 products measured slower that way (2.92 against 2.80
-    // ms) and stay on s.
+    // before the combine), the longer of the two on s.  What that gains is the launches' tails,
+    // 2 to 6%: a wide workgroup and a narrow one do not share a CU (252 registers of the wide
+    // tile's eight waves fill it), so that side by side the two parts take about the sum of
+    // their times.  (Two streams against one, K2 shape, bf16 rows: 250 tokens 1540 and 1641 us,
+    // 700 2019 and 2145, 1000 2338 and 2384, 2048 3226 and 3300, 4096 5543 and 5459; latent 300
+    // 3090 and 3180, 1100 4986 and 5111, 2048 7427 and 7492.)  The MXFP8 products, all on tiles
+    // of four waves, measured slower that way and stay on s.
     const bool split = SI > 0 && !mx && !one;
     hipStream_t st[2] = {s, s};                          // classes 0 and 1, class 2
     if (split) {
