@@ -1,6 +1,6 @@
-"""LatentMoE layers whose latent width is above the hidden size, in prefill: the routed rows
+"""LatentMoE layers whose latent width is above the hidden size: in prefill the routed rows
 (latent floats each) and the shared expert's rows (hidden floats each) share one buffer and
-are written on two streams.  On the library's shared expert (bf16 rows, 2 * n_shared * inter
+are written on two streams; decode calls of one to eight tokens beside them.  On the library's shared expert (bf16 rows, 2 * n_shared * inter
 <= hidden) and on the framework's own, in the exact and the MXFP8 mode, against the oracle
 (ko_moe, ko_moe_mx).  Relative L2 below 2e-5, the activations' 2^-17 (hi + lo) on each of the
 five products and fp32 sums of up to 768 terms (their square root times 2^-24 in practice)."""
@@ -26,7 +26,7 @@ def wide_layer(H, LT, I, NS):
 def test_latent_above_hidden(torch, k3x, H, LT, I, NS, bf16):
     L = wide_layer(H, LT, I, NS)
     layer = bank_layer(k3x, L)
-    for T in (9, 40, 200):
+    for T in (1, 2, 5, 8, 9, 40, 200):
         x = L.x(T, bf16=bf16, stream_sub=T)
         o, oi, _, _ = L.oracle_moe(x)
         out, idx, _ = dev_forward(torch, k3x, layer, x, bf16=bf16)
